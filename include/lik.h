@@ -123,6 +123,7 @@ typedef struct {
 #define LIK_NORMALIZE_Q 4u /* normalise query tokens only (docs already unit rows, e.g. decoded PLAID) */
 #define LIK_NORMALIZE_D 8u /* normalise doc tokens only (queries pre-normalised, e.g. a projection head) */
 #define LIK_BIAS_16 16u /* lik_maxsim_from_hidden: bias holds d_out values of Q's 16-bit dtype, not fp32 */
+#define LIK_PER_TOKEN 64u /* lik_quantize_fp8: one scale per row instead of one per tensor */
 #define LIK_TOKEN_RECORDS 32u /* lik_plaid_maxsim_qc: token_inv points at lik_plaid_token_t records */
 
 /*
@@ -401,6 +402,18 @@ int lik_topk_select(const float* scores, int64_t rows, int64_t n, int64_t ld, in
                     const float* prev_scores, const int64_t* prev_idx, int64_t prev_k,
                     int64_t prev_ld, int64_t k, int largest, float* out_scores, int64_t* out_idx,
                     int64_t out_ld, void* workspace, size_t workspace_bytes, lik_stream_t stream);
+
+/*
+ * fp8 (OCP e4m3fn) quantisation of x [rows, dim] (contiguous, bf16 / fp16 /
+ * fp32): scale = max(amax, 1e-6) / 448 in fp32, out = e4m3(clamp(x / scale)),
+ * round to nearest even. With LIK_PER_TOKEN scale is [rows], else one value.
+ * dim is a multiple of 8 (fp32: 4) elements and with LIK_PER_TOKEN at most
+ * 1024 (fp32: 512); x is 16-byte and out 8-byte aligned (LIK_ERR_UNSUPPORTED
+ * otherwise). Replaces fp8.py:35-59.
+ */
+size_t lik_quantize_fp8_workspace_size(uint32_t flags);
+int lik_quantize_fp8(const void* x, int32_t dtype, int64_t rows, int32_t dim, uint32_t flags, void* out, float* scale,
+                     void* workspace, size_t workspace_bytes, lik_stream_t stream);
 
 /*
  * Allocation-free scoring. No counterpart in the reference: this entry point

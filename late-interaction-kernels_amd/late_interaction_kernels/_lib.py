@@ -31,6 +31,7 @@ LIK_NORMALIZE_Q = 4
 LIK_NORMALIZE_D = 8
 LIK_BIAS_16 = 16
 LIK_TOKEN_RECORDS = 32
+LIK_PER_TOKEN = 64
 
 
 def norm_flags(norm: int) -> int:
@@ -73,6 +74,8 @@ EXPORTED_SYMBOLS = (
     "lik_plaid_token_records",
     "lik_plaid_maxsim_qc",
     "lik_plaid_maxsim_qc_workspace_size",
+    "lik_quantize_fp8",
+    "lik_quantize_fp8_workspace_size",
 )
 
 _p = ctypes.c_void_p
@@ -222,6 +225,10 @@ def load() -> ctypes.CDLL:
     lib.lik_plaid_maxsim_qc.argtypes = [P(LikSeqs), P(LikPlaidDocs), _p, ctypes.c_uint32, _p, _i64, _i64, _p,
                                         ctypes.c_size_t, P(LikLaunchOpts), _p]
     lib.lik_plaid_maxsim_qc.restype = ctypes.c_int
+    lib.lik_quantize_fp8_workspace_size.argtypes = [ctypes.c_uint32]
+    lib.lik_quantize_fp8_workspace_size.restype = ctypes.c_size_t
+    lib.lik_quantize_fp8.argtypes = [_p, _i32, _i64, _i32, ctypes.c_uint32, _p, _p, _p, ctypes.c_size_t, _p]
+    lib.lik_quantize_fp8.restype = ctypes.c_int
     _lib = lib
     return lib
 
@@ -241,6 +248,20 @@ def require_gpu(*tensors: torch.Tensor | None) -> None:
             )
     if getattr(torch.version, "hip", None) is None:
         raise RuntimeError("late_interaction_kernels (MI355X build) needs a ROCm build of PyTorch")
+
+
+def plain_op(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel may stand in for a chain of torch operators on these
+    tensors: GPU tensors of torch's own class, no gradient or forward-mode
+    tangent to carry, nothing tracing, batching or intercepting the operators."""
+    if any(type(t) not in (torch.Tensor, torch.nn.Parameter) or t.device.type != "cuda" for t in tensors):
+        return False
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return False
+    if torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.maybe_current_level() is not None:
+        return False
+    return not (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                or torch.jit.is_tracing() or torch.compiler.is_compiling())
 
 
 def stream_of(t: torch.Tensor) -> int:

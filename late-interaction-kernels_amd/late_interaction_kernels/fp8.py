@@ -15,6 +15,7 @@ from __future__ import annotations
 
 import torch
 
+from . import _lib
 from ._core import dense_maxsim
 from .autograd import _validate_devices
 
@@ -23,11 +24,39 @@ _E4M3 = getattr(torch, "float8_e4m3fn", None)
 _E5M2 = getattr(torch, "float8_e5m2", None)
 
 
+def _quantize_kernel(X: torch.Tensor, dtype: torch.dtype, per_token: bool):
+    """One pass over ``X`` (two per tensor) in ``lik_quantize_fp8``, with the
+    bytes and scales of the operator chain below; ``None`` where the kernel does
+    not apply (other dtypes and row widths, unaligned or non-contiguous X,
+    gradients, tracing, CPU tensors)."""
+    if dtype != _E4M3 or X.dtype not in (torch.bfloat16, torch.float16, torch.float32):
+        return None
+    if X.dim() == 0 or X.numel() == 0 or not _lib.plain_op(X) or not X.is_contiguous():
+        return None
+    epc, d = 16 // X.element_size(), X.shape[-1]
+    if d % epc or (per_token and d > 128 * epc) or d > 0x7FFFFFFF or X.data_ptr() % 16:
+        return None
+    flags = _lib.LIK_PER_TOKEN if per_token else 0
+    out = torch.empty(X.shape, device=X.device, dtype=dtype)
+    scale = torch.empty(X.shape[:-1] if per_token else (), device=X.device, dtype=torch.float32)
+    lib = _lib.load()
+    nbytes = lib.lik_quantize_fp8_workspace_size(flags)
+    ws = _lib.workspace(nbytes, X.device)
+    with torch.cuda.device(X.device):
+        rc = lib.lik_quantize_fp8(X.data_ptr(), _lib.DTYPE_CODE[X.dtype], X.numel() // d, d, flags, out.data_ptr(),
+                                  scale.data_ptr(), _lib.ptr(ws), nbytes, _lib.stream_of(out))
+    _lib.check(rc, "lik_quantize_fp8")
+    return out, scale
+
+
 def quantize_fp8_per_tensor(X: torch.Tensor, dtype: torch.dtype | None = None) -> tuple[torch.Tensor, torch.Tensor]:
     """Quantize with one fp32 scale; dequantize as ``X_fp8.float() * scale``."""
     dtype = dtype or _E4M3
     if X.numel() == 0:
         return X.to(dtype), torch.ones((), device=X.device, dtype=torch.float32)
+    done = _quantize_kernel(X, dtype, False)
+    if done is not None:
+        return done
     amax = X.abs().amax().clamp_min(1e-6).to(torch.float32)
     scale = amax / _FP8_E4M3_MAX
     X_fp8 = (X.to(torch.float32) / scale).clamp(-_FP8_E4M3_MAX, _FP8_E4M3_MAX).to(dtype)
@@ -37,6 +66,9 @@ def quantize_fp8_per_tensor(X: torch.Tensor, dtype: torch.dtype | None = None) -
 def quantize_fp8_per_token(X: torch.Tensor, dtype: torch.dtype | None = None) -> tuple[torch.Tensor, torch.Tensor]:
     """Quantize each row (last axis) with its own scale; scale has shape ``X.shape[:-1]``."""
     dtype = dtype or _E4M3
+    done = _quantize_kernel(X, dtype, True)
+    if done is not None:
+        return done
     amax = X.abs().amax(dim=-1).clamp_min(1e-6).to(torch.float32)
     scale = amax / _FP8_E4M3_MAX
     X_fp8 = (X.to(torch.float32) / scale.unsqueeze(-1)).clamp(-_FP8_E4M3_MAX, _FP8_E4M3_MAX).to(dtype)
