@@ -60,7 +60,8 @@ constexpr bool two_wg_per_cu() {
   // 16-bit ones, and a tile holds only two k-steps of MFMA work, so more
   // column blocks per wave amortise the per-tile work (+30% measured)
   return W == 4 && (NSUB == 4 || (NSUB == 6 && EK == EK_FP8)) && SRC == SRC_DENSE &&
-         (EK == EK_BF16 || EK == EK_F16 || EK == EK_FP8) && (FEAT & (F_ARGMAX | F_NORM | F_TS | F_MASK)) == 0;
+         (EK == EK_BF16 || EK == EK_F16 || EK == EK_FP8) &&
+         (FEAT & (F_ARGMAX | F_NORM | F_MASK | (EK == EK_FP8 ? 0 : F_TS))) == 0;
 }
 // Workgroups per CU of those kernels (fp8 would nearly fit three, but spills
 // at 168 VGPRs and measures slower).
@@ -164,10 +165,9 @@ __global__ void __launch_bounds__(W * 64)
   if constexpr (SRC == SRC_PLAID) {
     for (int i = tid; i < 256; i += NT) s_bw[i] = i < p.pl.nb ? p.pl.bw[i] : 0.f;
   }
-  // Row scales start at 0 (the first iteration's epilogue runs on the
-  // -inf-initialised accumulator set; the epilogue keeps -inf rows at -inf
-  // whatever their scale).
-  for (int i = tid; i < 4 * 32; i += NT) s_rs[i >> 5][i & 31] = 0.f;
+  // Row scales start at 1: the first iteration's epilogue runs on the
+  // -inf-initialised accumulator set, and -inf rows have scale 1 (see commit).
+  for (int i = tid; i < 4 * 32; i += NT) s_rs[i >> 5][i & 31] = 1.f;
 
   // ---------------- document range and tile cursor ----------------
   const int64_t jl0 = r * (int64_t)p.R;
@@ -656,7 +656,11 @@ __global__ void __launch_bounds__(W * 64)
             *(u32x4*)(rowp + cc * 16) = v;
           }
           if constexpr (kRowScaleEpi) {
-            if (cc == 0) s_rs[rslot][row] = (f_norm ? inv_norm(ss) : 1.f) * (f_ts ? sts[S][i] : 1.f);
+            // rows that are not scored (past the doc end, dropped by the mask)
+            // get scale 1, so their -inf stays -inf without a test per element
+            bool live = row < d.nv;
+            if constexpr ((FEAT & F_MASK) != 0) live = live && !(d.holes && !((sm[S] >> (row & 31)) & 1u));
+            if (cc == 0) s_rs[rslot][row] = live ? (f_norm ? inv_norm(ss) : 1.f) * (f_ts ? sts[S][i] : 1.f) : 1.f;
           }
         }
       } else {
@@ -883,19 +887,19 @@ __global__ void __launch_bounds__(W * 64)
     }
     if constexpr (kRowScaleEpi) {
       if (row_scale) {
-        f32x4 sc[4];
+        // (one group of four rows' scales at a time: 4 registers)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sc[j] = *(const f32x4*)&s_rs[rslot][8 * j + 4 * h];
+        for (int j = 0; j < 4; ++j) {
+          const f32x4 sc = *(const f32x4*)&s_rs[rslot][8 * j + 4 * h];
 #pragma unroll
-        for (int sub = 0; sub < NSUB; ++sub)
+          for (int sub = 0; sub < NSUB; ++sub) {
+            float v[4];
 #pragma unroll
-          for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              // invalid rows hold -inf and may have a 0 or NaN scale: they stay -inf
-              const float a = acc[P][sub][4 * j + e];
-              m[sub] = max_nan(m[sub], a == NEG_INF ? NEG_INF : a * sc[j][e]);
-            }
+            for (int e = 0; e < 4; ++e) v[e] = acc[P][sub][4 * j + e] * sc[e];
+            m[sub] = max_nan(m[sub], max_nan(v[0], v[1]));
+            m[sub] = max_nan(m[sub], max_nan(v[2], v[3]));
+          }
+        }
         return;
       }
     }

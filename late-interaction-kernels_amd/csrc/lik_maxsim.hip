@@ -456,14 +456,20 @@ bool prenorm_docs(const lik_seqs_t* Q, const lik_seqs_t* D, uint32_t flags, cons
          (Q->dtype == LIK_BF16 || Q->dtype == LIK_F16) && D->len > 0;
 }
 
-// The plan of a scoring call: the two-workgroup 4 x 4 block is preferred when
-// the tile loop does no doc-side work (no doc normalise left in the kernel,
-// no argmax, no token scales).
+// The plan of a scoring call: the two-workgroup 4 x 4 block (fp8 also 4 x 6)
+// is preferred when the tile loop does no doc-side work (no doc normalise left
+// in the kernel, no argmax). fp8 rows with their own scales count as plain at
+// 65 .. 128 dims, where the kernel is compiled for exactly that: the scales
+// cost one multiply per element of the epilogue (64 x 24 query tokens against
+// 1000 x 1030 rows of d = 128: 494 us on 8 x 4, which also left a third of its
+// second 1024-column group empty, 239 us on 4 x 6). At other widths the
+// all-features kernel takes one workgroup per CU either way and keeps 8 x 4.
 int plan_call(const lik_seqs_t* Q, const lik_seqs_t* D, uint32_t flags, bool argmax, Plan& pl, bool& prenorm,
               const lik_launch_opts_t* opts, bool allow_prenorm = true) {
   const bool kd = (flags & LIK_KD_LAYOUT) != 0;
   const int min_w = ((norm_bits(flags) & 2) || argmax) ? 4 : 1;
-  const bool plain = !argmax && !row_scale(Q) && !row_scale(D);
+  const bool scaled = row_scale(Q) || row_scale(D);
+  const bool plain = !argmax && (!scaled || pick_dpad(Q->dtype, Q->dim) == 128);
   int rc = make_plan(Q->dtype, Q->dim, Q->n, Q->len, kd, pl, min_w, plain, opts);
   if (rc != LIK_OK) return rc;
   prenorm = prenorm_docs(Q, D, flags, pl, allow_prenorm);
