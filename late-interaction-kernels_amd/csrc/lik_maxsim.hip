@@ -971,6 +971,59 @@ int lik_plaid_maxsim_ex(const lik_seqs_t* Q, const lik_plaid_docs_t* docs, uint3
     return timed_launch(s, opts, [&] { return launch_plaid_stream(ek, cdk, sdp, nsub, p, s); });
   }
 
+  // Larger query blocks, 16-bit centroids, rows of up to 128 dims: four decoded
+  // tiles per barrier (lik_plaid_block.hip). plaid_variant 3 or a forced
+  // column block keeps the tile kernel, which takes everything else.
+  if (Q->len >= 1 && Q->len <= 512 && (sdp == 64 || sdp == 128) && docs->centroid_dtype != LIK_F32 && variant != 3 &&
+      !(opts && opts->col_waves > 0)) {
+    Params p{};
+    p.q = to_dev(*Q);
+    p.pl.codes = docs->codes;
+    p.pl.res = docs->residuals;
+    p.pl.cu = docs->cu_seqlens;
+    p.pl.lengths = docs->lengths;
+    p.pl.n = docs->n;
+    p.pl.L = docs->max_len;
+    p.pl.codes_sn = docs->codes_stride_n;
+    p.pl.res_st = docs->res_stride_tok;
+    p.pl.cent = (const char*)docs->centroids;
+    p.pl.cent_sb = docs->cent_stride * ceb;
+    p.pl.ncent = docs->n_centroids;
+    p.pl.bw = docs->bucket_weights;
+    p.pl.nb = docs->n_buckets;
+    p.pl.nbits = docs->nbits;
+    p.normalize = norm_bits(flags);
+    p.out_scale = 1.f;
+    p.out = out;
+    p.osq = out_stride_q;
+    p.osd = out_stride_d;
+    const int cols = Q->n * Q->len > 256 ? 512 : 256;
+    p.nc = 1;
+    p.nunits = Q->n;
+    p.LU = (int)Q->len;
+    p.QPG = cols / p.LU;
+    p.ngroups = (Q->n + p.QPG - 1) / p.QPG;
+    p.ndocs_pg = docs->n;
+    // One workgroup per CU at a time, ~11 us of prologue and pipeline fill
+    // each: whole rounds of 256 workgroups of about 18 docs (4096 docs of 225
+    // tokens, 16 queries: 16 docs per workgroup 146 us, 8: 158, 4: 186, 32:
+    // 234; 20,000 docs: 16 docs 662 us, 27: 699, 64: 910).
+    const int64_t units = docs->n * p.ngroups;
+    const int64_t rounds = units > 256 * 27 ? (units + 256 * 9) / (256 * 18) : 1;
+    int64_t R = (units + 256 * rounds - 1) / (256 * rounds);
+    if (opts && opts->docs_per_wg > 0) R = opts->docs_per_wg;
+    R = R < 1 ? 1 : (R > docs->n ? docs->n : R);
+    p.R = (int)(R > 512 ? 512 : R);
+    p.NR = (docs->n + p.R - 1) / p.R;
+    p.xcd_map = p.NR >= 8 ? 1 : 0;
+    const int64_t nb = p.xcd_map ? p.ngroups * ((p.NR + 7) / 8) * 8 : p.ngroups * p.NR;
+    return timed_launch((hipStream_t)stream, opts, [&] {
+      return launch_plaid_block(Q->dtype == LIK_F16 ? EK_F16 : EK_BF16,
+                                docs->centroid_dtype == LIK_F16 ? EK_F16 : EK_BF16, sdp, cols, p, nb,
+                                (hipStream_t)stream);
+    });
+  }
+
   Plan pl;
   // PLAID tiles carry the decode VALU work: at least 4 waves share each tile
   // even when the query block would fit one wave's columns.

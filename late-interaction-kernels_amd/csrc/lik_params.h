@@ -125,6 +125,8 @@ bool q1_eligible(int dt, const Plan& pl, const Params& p);
 int launch_q1(int dt, const Plan& pl, const Params& p, hipStream_t s);
 // Few-query PLAID scoring, one wavefront per (query group, doc range): lik_plaid_stream.hip.
 int launch_plaid_stream(int ek, int cd, int dpad, int nsub, const Params& p, hipStream_t s);
+// PLAID decode + MaxSim for blocks of 256 / 512 query tokens: lik_plaid_block.hip.
+int launch_plaid_block(int ek, int cd, int dpad, int cols, const Params& p, int64_t nb, hipStream_t s);
 // rows wider than the tile kernel takes (lik_wide.hip): one wave per (query, doc)
 int launch_maxsim_wide(int dtype, const Params& p, hipStream_t s);
 // training forward (argmax output), lik_inst_train_*.hip
