@@ -29,7 +29,9 @@
 //   (grad_d_kd_kernel: a doc's winners come from <= 64 pairs, so one
 //   workgroup per doc) and cross products with >= 8192
 //   (query, token) pairs (grad_d_sorted_kernel over the winner entries
-//   radix-sorted by doc row).
+//   radix-sorted by doc row). 16-bit rows of up to 128 dims have their own
+//   kernels, 16 bytes a lane: grad_q_rows_kernel, and grad_d_doc_kernel for
+//   cross products of up to 12288 pairs.
 // Packed queries: the wave of (i, s) exits when s is past query i's length;
 // rows are addressed through cu_q (reference varlen.py:143-263).
 // Pair lists (reference score_pairs.py:344-420): the score units are pairs p =
@@ -97,7 +99,13 @@ struct BwdParams {
   // row-block kernel): entries row_vals[row_ptr[r] .. row_ptr[r + 1]) of row r
   const int32_t* row_ptr;
   const int32_t* row_vals;
+  // every Q / D row starts below 2^32 16-byte units from the first, and the
+  // gradient rows are whole 16-byte chunks: the 16-bytes-a-lane kernels apply
+  bool q_units, d_units;
 };
+
+// most (query, token) pairs per doc that grad_d_doc_kernel sorts in LDS
+constexpr int64_t kDocPairs = 12288;
 
 // inv[r] = 1 / max(||row r||, 1e-12) for rows r = i*L + t of a [n, L, dim]
 // tensor: LPR lanes per row, each summing 16-byte chunks, then an xor-shuffle
@@ -724,12 +732,374 @@ __global__ void __launch_bounds__(256) grad_d_sorted_kernel(const BwdParams bp) 
   }
 }
 
+// ---- 16-bit rows of up to 128 dims: 8 DPL lanes per row, 16 bytes a lane ----
+//
+// The one-wavefront-per-row kernels above spend about 50 instructions on each
+// winning row (4 bytes a lane, the row's address and scale read out of lanes
+// one by one), so they are bound by instruction issue. Here a lane holds 8
+// dims: a wavefront adds 8 / DPL winning rows at once, one load and 16
+// arithmetic instructions each time. Every element's sum keeps its order, and
+// the dot product of the normalise Jacobian the association of wave_sum, so
+// the gradients are bitwise those of the kernels above. (256 queries of 32
+// tokens x 256 docs of 300, d = 128: grad_q 212 -> 43 us for 537 MB of winning
+// rows out of L2 and the memory-side cache, 12.5 TB/s.)
+
+template <int EK>
+__device__ __forceinline__ void unpack8(const u32x4& v, float* x) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (EK == EK_BF16) {
+      x[2 * i] = bf16lo_to_f32(v[i]);
+      x[2 * i + 1] = bf16hi_to_f32(v[i]);
+    } else {
+      x[2 * i] = f16_to_f32((uint16_t)(v[i] & 0xffffu));
+      x[2 * i + 1] = f16_to_f32((uint16_t)(v[i] >> 16));
+    }
+  }
+}
+template <int EK>
+__device__ __forceinline__ u32x4 pack8(const float* x) {
+  u32x4 v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (EK == EK_BF16)
+      v[i] = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)x[2 * i], (__bf16)x[2 * i + 1]});
+    else
+      v[i] = f32_to_f16_bits(x[2 * i]) | (f32_to_f16_bits(x[2 * i + 1]) << 16);
+  }
+  return v;
+}
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_row(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+}
+// Lane L of the row's lanes, to all of them.
+template <int DPL, int L>
+__device__ __forceinline__ uint32_t row_bcast(uint32_t v) {
+  if constexpr (DPL == 2) return dpp_row<0x150 + L>(v);  // row_newbcast
+  else return (uint32_t)__shfl((int)v, (int)((threadIdx.x & 56) + L));
+}
+
+// <g, xh> over a row's 64 DPL elements (8 a lane), summed as wave_sum sums
+// lanes of DPL elements: lanes 32, 16, 8, 4, 2, 1 apart in turn.
+template <int DPL>
+__device__ __forceinline__ float row_dot(const float* g, const float* xh) {
+  constexpr int NP = 8 / DPL;
+  float p[NP];
+#pragma unroll
+  for (int r = 0; r < NP; ++r) {
+    p[r] = fmaf(g[DPL * r], xh[DPL * r], 0.f);
+    if constexpr (DPL == 2) p[r] = fmaf(g[2 * r + 1], xh[2 * r + 1], p[r]);
+    if constexpr (DPL == 2) {
+      // rotations by 8, 4, 2, 1: the lanes they bring hold what the xor partners hold
+      p[r] += __uint_as_float(dpp_row<0x128>(__float_as_uint(p[r])));
+      p[r] += __uint_as_float(dpp_row<0x124>(__float_as_uint(p[r])));
+      p[r] += __uint_as_float(dpp_row<0x122>(__float_as_uint(p[r])));
+      p[r] += __uint_as_float(dpp_row<0x121>(__float_as_uint(p[r])));
+    } else {
+#pragma unroll
+      for (int o = 4; o >= 1; o >>= 1) p[r] += __shfl_xor(p[r], o);
+    }
+  }
+  if constexpr (DPL == 2) return (p[0] + p[2]) + (p[1] + p[3]);
+  else return ((p[0] + p[4]) + (p[2] + p[6])) + ((p[1] + p[5]) + (p[3] + p[7]));
+}
+
+// The Jacobian of x / ||x|| on a finished gradient row, inv = 1 / ||x||.
+template <int EK, int DPL>
+__device__ __forceinline__ void row_jacobian(float* g, const char* row, bool live, int q, float inv) {
+  float xh[8];
+  const u32x4 v = live ? *(const u32x4*)(row + q * 16) : u32x4{0u, 0u, 0u, 0u};
+  unpack8<EK>(v, xh);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) xh[k] *= inv;
+  const float dot = row_dot<DPL>(g, xh);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) g[k] = (g[k] - dot * xh[k]) * inv;
+}
+
+constexpr uint32_t kNoRow = 0xffffffffu;  // "no winner" among row offsets in 16-byte units
+
+// grad_q_kernel for these rows: each group of 8 DPL lanes takes a query token,
+// loads the argmax, G and scale of 8 DPL units at once (the next ones' while
+// these are added) and adds the winning rows in unit order, 8 loads at a time.
+template <int EK, int DPL>
+__global__ void __launch_bounds__(256) grad_q_rows_kernel(const BwdParams bp) {
+  constexpr int LPR = 8 * DPL, TPW = 64 / LPR;  // lanes per row, tokens per wavefront
+  const int lane = threadIdx.x & 63, q = lane & (LPR - 1);
+  const int64_t nwt = bp.nq * bp.lq;
+  const int64_t per = (nwt + TPW - 1) / TPW;  // wavefronts per doc split
+  const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (wave >= per * bp.qsplit) return;
+  const int64_t c = wave / per;
+  const int64_t w = (wave - c * per) * TPW + lane / LPR;
+  if (w >= nwt) return;
+  const int64_t i = w / bp.lq, s = w - i * bp.lq;
+  const int64_t qr = grad_q_row(bp, i, s, w);
+  if (qr < 0) return;
+  const int64_t j0 = bp.kd ? i * bp.ndoc_pg : 0;
+  int64_t nu = bp.ndoc_pg, u0 = 0;
+  if (bp.q_ptr) {
+    u0 = bp.q_ptr[i];
+    nu = (int64_t)bp.q_ptr[i + 1] - u0;
+  }
+  int64_t ub = 0, ue = nu;
+  if (bp.qsplit > 1) {
+    ub = c * bp.qchunk;
+    ue = ub + bp.qchunk < nu ? ub + bp.qchunk : nu;
+  }
+  const bool live = q * 8 < bp.dim;
+  auto load_units = [&](int64_t c0, uint32_t& off, float& sc) {
+    off = kNoRow;
+    sc = 0.f;
+    const int64_t jl = c0 + q;
+    if (jl >= ue) return;
+    int a;
+    float g;
+    int64_t jd;
+    if (bp.q_ptr) {
+      const int64_t pr = bp.q_list[u0 + jl];
+      a = bp.amax[pr * bp.lq + s];
+      g = bp.grad[pr];
+      jd = bp.pair_d[pr];
+    } else {
+      a = bp.amax[(i * bp.ndoc_pg + jl) * bp.lq + s];
+      g = bp.grad[i * bp.ld_g + jl];
+      jd = j0 + jl;
+    }
+    if (a < 0 || g == 0.f) return;
+    sc = bp.dinv ? g * bp.dinv[jd * bp.ld + a] : g;  // dinv only for padded docs
+    const int64_t b = bp.d_cu ? ((int64_t)bp.d_cu[jd] + a) * bp.d_sl : jd * bp.d_sn + (int64_t)a * bp.d_sl;
+    off = (uint32_t)(b >> 4);
+  };
+  float acc[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) acc[k] = 0.f;
+  uint32_t off, off_n;
+  float sc, sc_n;
+  load_units(ub, off, sc);
+  for (int64_t c0 = ub; c0 < ue; c0 += LPR) {
+    load_units(c0 + LPR, off_n, sc_n);
+    auto batch = [&](auto B) {
+      u32x4 v[8];
+      float cs[8];
+      auto one = [&](auto K) {
+        constexpr int k = decltype(K)::value, l = decltype(B)::value * 8 + k;
+        const uint32_t o = row_bcast<DPL, l>(off);
+        cs[k] = __uint_as_float(row_bcast<DPL, l>(__float_as_uint(sc)));
+        v[k] = u32x4{0u, 0u, 0u, 0u};
+        if (o != kNoRow && live) v[k] = *(const u32x4*)(bp.d + ((uint64_t)o << 4) + q * 16);
+      };
+      one(std::integral_constant<int, 0>{});
+      one(std::integral_constant<int, 1>{});
+      one(std::integral_constant<int, 2>{});
+      one(std::integral_constant<int, 3>{});
+      one(std::integral_constant<int, 4>{});
+      one(std::integral_constant<int, 5>{});
+      one(std::integral_constant<int, 6>{});
+      one(std::integral_constant<int, 7>{});
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        float x[8];
+        unpack8<EK>(v[k], x);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = fmaf(cs[k], x[e], acc[e]);
+      }
+    };
+    batch(std::integral_constant<int, 0>{});
+    if constexpr (DPL == 2) batch(std::integral_constant<int, 1>{});
+    off = off_n;
+    sc = sc_n;
+  }
+  if (bp.qsplit > 1) {
+    float* part = bp.gq_part + (c * nwt + w) * (64 * DPL) + q * 8;
+    *(f32x4*)part = f32x4{acc[0], acc[1], acc[2], acc[3]};
+    *(f32x4*)(part + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]};
+    return;
+  }
+  const bool keep = !bp.qmask || bp.qmask[i * bp.qm_sn + s * bp.qm_sl] != 0;
+  if (bp.qinv) {
+    const char* qrow = bp.q_cu ? bp.q + qr * bp.q_sl : bp.q + i * bp.q_sn + s * bp.q_sl;
+    row_jacobian<EK, DPL>(acc, qrow, live, q, bp.qinv[qr]);
+  }
+  if (live) *(u32x4*)(bp.gq + (qr * bp.dim + q * 8) * 2) = keep ? pack8<EK>(acc) : u32x4{0u, 0u, 0u, 0u};
+}
+
+// grad_D of a cross product (padded docs and queries) for these rows: one
+// workgroup per (doc j, range of its rows). The (query, token) pairs f = i Lq + s
+// whose winner lies in the range are sorted by row in LDS, stably (each
+// wavefront counts, then places, its own contiguous share of the pairs), so a
+// row's entries stay in increasing f, the order every grad_D kernel adds them
+// in; then each group of 8 DPL lanes adds a row's entries, takes the Jacobian
+// and stores it, rows without entries as zeros.
+//
+// Against keys + device radix sort + bucket pointers + one wavefront per row
+// (grad_d_sorted_kernel, which more pairs still take) this is one launch that
+// reads the argmax once and writes nothing but the gradient: 8192 pairs per
+// doc, 256 docs of 300 rows: 215 us in 12 launches -> 43 us. 2048 pairs and
+// fewer run four-wavefront workgroups, several per CU; above 12288 pairs the
+// sorted entries (8 bytes each) no longer fit the LDS beside the counters.
+template <int EK, int DPL, int NW, int MAXP, int MAXROWS>
+__global__ void __launch_bounds__(NW * 64) grad_d_doc_kernel(const BwdParams bp, int nsplit, int rows_per) {
+  constexpr int NT = NW * 64, CH = MAXP / NT, RPT = (MAXROWS + NT - 1) / NT, LPR = 8 * DPL;
+  __shared__ __attribute__((aligned(16))) uint2 s_ent[MAXP];  // {query row offset / 16, scale bits}, by row
+  __shared__ __attribute__((aligned(16))) uint16_t s_cnt[NW][MAXROWS];
+  __shared__ int s_ptr[MAXROWS + 1];
+  __shared__ int s_tot[NW];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int64_t j = blockIdx.x / nsplit;
+  const int t0 = (int)(blockIdx.x - j * nsplit) * rows_per;
+  const int nrows = (int)(bp.ld - t0 < rows_per ? bp.ld - t0 : rows_per);
+  if (nrows <= 0) return;
+  for (int k = tid; k < NW * MAXROWS / 2; k += NT) ((uint32_t*)s_cnt)[k] = 0u;
+  const int np = (int)(bp.nq * bp.lq);
+  const int share = (np + NT - 1) / NT * 64;  // pairs per wavefront
+  int key[CH];
+  float sc[CH];
+  uint32_t off[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int f = wv * share + c * 64 + lane;
+    key[c] = -1;
+    sc[c] = 0.f;
+    off[c] = 0u;
+    if (c * 64 < share && f < np) {
+      const int i = f / (int)bp.lq, s = f - i * (int)bp.lq;
+      const float g = bp.grad[i * bp.ld_g + j];
+      const int a = bp.amax[((int64_t)i * bp.nd + j) * bp.lq + s];
+      const bool keep = !bp.qmask || bp.qmask[i * bp.qm_sn + s * bp.qm_sl] != 0;
+      sc[c] = bp.qinv ? g * bp.qinv[f] : g;
+      off[c] = (uint32_t)((i * bp.q_sn + s * bp.q_sl) >> 4);
+      if (a >= t0 && a < t0 + nrows && g != 0.f && keep) key[c] = a - t0;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+    if (key[c] >= 0) atomicAdd((uint32_t*)s_cnt[wv] + (key[c] >> 1), 1u << (16 * (key[c] & 1)));
+  __syncthreads();
+  // row pointers, and each wavefront's first position in each row
+  int cnt[RPT], mine = 0;
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) {
+    const int row = tid * RPT + r;
+    cnt[r] = 0;
+    if (row < nrows)
+      for (int w = 0; w < NW; ++w) cnt[r] += s_cnt[w][row];
+    mine += cnt[r];
+  }
+  int incl = mine;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int t = __shfl_up(incl, o);
+    if (lane >= o) incl += t;
+  }
+  if (lane == 63) s_tot[wv] = incl;
+  __syncthreads();
+  int base = incl - mine;
+  for (int w = 0; w < wv; ++w) base += s_tot[w];
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) {
+    const int row = tid * RPT + r;
+    if (row < nrows) {
+      s_ptr[row] = base;
+      int b = base;
+      for (int w = 0; w < NW; ++w) {
+        const int n = s_cnt[w][row];
+        s_cnt[w][row] = (uint16_t)b;
+        b += n;
+      }
+      base = b;
+      if (row == nrows - 1) s_ptr[nrows] = base;
+    }
+  }
+  __syncthreads();
+  const int kbits = 32 - __builtin_clz(nrows);  // keys are below nrows
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    if (c * 64 >= share) break;
+    // lanes with this lane's key: their number below it is its rank
+    uint64_t same = __ballot(key[c] >= 0);
+    for (int b = 0; b < kbits; ++b) {
+      const bool on = (key[c] >> b) & 1;
+      const uint64_t m = __ballot(on);
+      same &= on ? m : ~m;
+    }
+    if (key[c] >= 0) {
+      const int rank = (int)__popcll(same & ((1ull << lane) - 1ull));
+      const int pos = s_cnt[wv][key[c]] + rank;
+      s_ent[pos] = uint2{off[c], __float_as_uint(sc[c])};
+      if (rank == 0) s_cnt[wv][key[c]] = (uint16_t)(pos + (int)__popcll(same));
+    }
+  }
+  __syncthreads();
+  const int q = lane & (LPR - 1);
+  const bool live = q * 8 < bp.dim;
+  for (int r = tid / LPR; r < nrows; r += NT / LPR) {
+    const int b = s_ptr[r], e = s_ptr[r + 1];
+    float g[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) g[k] = 0.f;
+    for (int k0 = b; k0 < e; k0 += 8) {
+      u32x4 v[8];
+      float cs[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        v[k] = u32x4{0u, 0u, 0u, 0u};
+        cs[k] = 0.f;
+        if (k0 + k < e) {
+          const uint2 en = s_ent[k0 + k];
+          cs[k] = __uint_as_float(en.y);
+          if (live) v[k] = *(const u32x4*)(bp.q + ((uint64_t)en.x << 4) + q * 16);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        float x[8];
+        unpack8<EK>(v[k], x);
+#pragma unroll
+        for (int d = 0; d < 8; ++d) g[d] = fmaf(cs[k], x[d], g[d]);
+      }
+    }
+    const int64_t t = t0 + r;
+    if (bp.dinv && e > b)
+      row_jacobian<EK, DPL>(g, bp.d + j * bp.d_sn + t * bp.d_sl, live, q, bp.dinv[j * bp.ld + t]);
+    if (live) *(u32x4*)(bp.gd + ((j * bp.ld + t) * bp.dim + q * 8) * 2) = pack8<EK>(g);
+  }
+}
+
+template <int EK, int DPL, int NW, int MAXP, int MAXROWS>
+int launch_grad_d_doc(const BwdParams& bp, int64_t want, hipStream_t s) {
+  // about `want` workgroups, each of at least 32 rows
+  int64_t split = (want + bp.nd - 1) / bp.nd;
+  const int64_t most = (bp.ld + 31) / 32, least = (bp.ld + MAXROWS - 1) / MAXROWS;
+  split = split < most ? split : most;
+  split = split > least ? split : least;
+  const int64_t rows = (bp.ld + split - 1) / split;
+  split = (bp.ld + rows - 1) / rows;
+  if (bp.nd * split > 0x7fffffffLL) return LIK_ERR_UNSUPPORTED;
+  hipLaunchKernelGGL((grad_d_doc_kernel<EK, DPL, NW, MAXP, MAXROWS>), dim3((unsigned)(bp.nd * split)), dim3(NW * 64), 0,
+                     s, bp, (int)split, (int)rows);
+  return hipGetLastError() == hipSuccess ? LIK_OK : LIK_ERR_LAUNCH;
+}
+
 template <int EK, int DPL>
 int launch_bwd(const BwdParams& bp, hipStream_t s) {
   constexpr int RB = grad_d_rows<DPL>();
   const int64_t nw = bp.nq * bp.lq;
   if (nw > 0) {
-    hipLaunchKernelGGL((grad_q_kernel<EK, DPL>), dim3((unsigned)((nw * bp.qsplit + 3) / 4)), dim3(256), 0, s, bp);
+    bool done = false;
+    if constexpr (EK != EK_F32 && DPL <= 2) {
+      if (bp.d_units) {
+        constexpr int TPW = 8 / DPL;
+        const int64_t nwv = (nw + TPW - 1) / TPW * bp.qsplit;
+        hipLaunchKernelGGL((grad_q_rows_kernel<EK, DPL>), dim3((unsigned)((nwv + 3) / 4)), dim3(256), 0, s, bp);
+        done = true;
+      }
+    }
+    if (!done)
+      hipLaunchKernelGGL((grad_q_kernel<EK, DPL>), dim3((unsigned)((nw * bp.qsplit + 3) / 4)), dim3(256), 0, s, bp);
     if (hipGetLastError() != hipSuccess) return LIK_ERR_LAUNCH;
     if (bp.qsplit > 1) {
       hipLaunchKernelGGL((grad_q_finish_kernel<EK, DPL>), dim3((unsigned)((nw + 3) / 4)), dim3(256), 0, s, bp);
@@ -747,6 +1117,14 @@ int launch_bwd(const BwdParams& bp, hipStream_t s) {
     if (bp.nd > 0x7fffffffLL) return LIK_ERR_UNSUPPORTED;
     hipLaunchKernelGGL((grad_d_kd_kernel<EK, DPL>), dim3((unsigned)bp.nd), dim3(256), 0, s, bp);
     return hipGetLastError() == hipSuccess ? LIK_OK : LIK_ERR_LAUNCH;
+  }
+  if constexpr (EK != EK_F32 && DPL <= 2) {
+    if (bp.gd && bp.q_units && !bp.kd && !bp.q_ptr && !bp.q_cu && !bp.d_cu && ((uintptr_t)bp.gd) % 16 == 0) {
+      const int64_t np = bp.nq * bp.lq;
+      if (np <= 2048) return launch_grad_d_doc<EK, DPL, 4, 2048, 512>(bp, 1024, s);
+      if (np <= 8192) return launch_grad_d_doc<EK, DPL, 16, 8192, 1024>(bp, 256, s);
+      if (np <= kDocPairs) return launch_grad_d_doc<EK, DPL, 16, kDocPairs, 1024>(bp, 256, s);
+    }
   }
   // packed docs: sum of lengths <= nd * ld, so nd * ld / RB blocks cover them
   const int64_t nb = !bp.gd ? 0 : bp.d_cu ? (bp.nd * bp.ld + RB - 1) / RB : bp.nd * ((bp.ld + RB - 1) / RB);
@@ -894,6 +1272,22 @@ static size_t grad_q_part_bytes(const lik_seqs_t* Q, const lik_seqs_t* D, uint32
   return (size_t)(split * Q->n * Q->len * 64 * dpl) * sizeof(float);
 }
 
+// Whether the 16-bytes-a-lane kernels can address this side's rows: 16-bit rows
+// of up to 128 dims (whole 16-byte chunks; checked by the callers), each
+// starting below 2^32 16-byte units. A packed side has at most n * len rows.
+static bool row_units(const lik_seqs_t* x) {
+  if ((x->dtype != LIK_BF16 && x->dtype != LIK_F16) || x->dim > 128 || x->n <= 0 || x->len <= 0) return false;
+  const int64_t last = x->cu_seqlens ? x->n * x->len * x->stride_l
+                                     : (x->n - 1) * x->stride_n + (x->len - 1) * x->stride_l;
+  return last >= 0 && last * 2 < ((int64_t)0xffffffff << 4);
+}
+
+// grad_d_doc_kernel takes the call: a padded cross product whose pairs fit its
+// LDS sort. (At and below 64 pairs per doc the KD kernel comes first.)
+static bool doc_kernel(const lik_seqs_t* Q, const lik_seqs_t* D, uint32_t flags) {
+  return !(flags & LIK_KD_LAYOUT) && !Q->cu_seqlens && !D->cu_seqlens && row_units(Q) && Q->n * Q->len <= kDocPairs;
+}
+
 // Sorted-entry grad_D (cross product, padded, many pairs per doc): keys and
 // values in and out, the row pointers, the sort's temporary storage.
 struct RowWs {
@@ -909,6 +1303,7 @@ static RowWs row_ws_layout(const lik_seqs_t* Q, const lik_seqs_t* D, uint32_t fl
   // worth it when a row block would rescan many pairs (measured: 8192 pairs
   // per doc 0.92 -> 0.81 ms, 65,920 2.65 -> 2.21 ms, but 4096 pairs over
   // 1030-token docs 0.45 -> 0.50 ms); 32-bit entry and row ids
+  if (doc_kernel(Q, D, flags)) return w;
   if (Q->n * Q->len < 8192 || n >= ((int64_t)1 << 31) || rows >= ((int64_t)1 << 31) - 1) return w;
   size_t o = 0;
   const size_t a = align256((size_t)n * 4);
@@ -985,6 +1380,8 @@ int lik_maxsim_backward(const float* grad, int64_t grad_ld, const lik_seqs_t* Q,
   if (((uintptr_t)Q->data) % 16 || ((uintptr_t)D->data) % 16 || (Q->dim * eb) % 16 || bp.q_sl % 16 || bp.d_sl % 16 ||
       bp.q_sn % 16 || bp.d_sn % 16)
     return LIK_ERR_UNSUPPORTED;
+  bp.q_units = doc_kernel(Q, D, flags);
+  bp.d_units = row_units(D) && (uintptr_t)grad_q % 16 == 0;
   bp.nq = Q->n;
   bp.lq = Q->len;
   bp.nd = D->n;
@@ -1114,6 +1511,7 @@ int lik_maxsim_pairs_backward(const float* grad, const lik_seqs_t* Q, const lik_
   bp.qm_sl = Q->mask_stride_l;
   bp.gq = (char*)grad_q;
   bp.gd = (char*)grad_d;
+  bp.d_units = row_units(D) && (uintptr_t)grad_q % 16 == 0;
   bp.nq = Q->n;
   bp.lq = Q->len;
   bp.nd = D->n;
