@@ -365,12 +365,11 @@ int make_plan(int dt, int dim, int64_t nq, int64_t lq, bool one_query_per_group,
   return LIK_OK;
 }
 
-// Docs per workgroup: aim for >= ~2048 workgroups so 256 CUs see several
-// waves of work, but keep at least a few docs per workgroup to amortise the
-// query-block load.
-// Docs per workgroup. dpad > 0: a dense MaxSim launch of that row width
-// (PLAID tiles pass 0: their workgroups are latency-bound, more of them help).
-int pick_R(int64_t ngroups, int64_t ndocs, int dpad, const lik_launch_opts_t* opts = nullptr) {
+// Docs per workgroup. dpad > 0: a dense MaxSim launch of that row width (PLAID
+// tiles pass 0: their workgroups are latency-bound, more of them help).
+// wg_cu > 0: a cross product whose workgroups share a CU wg_cu at a time.
+int pick_R(int64_t ngroups, int64_t ndocs, int dpad, const lik_launch_opts_t* opts = nullptr, int wg_cu = 0,
+           bool packed = false) {
   const int64_t target = 2048;
   int64_t R = (ndocs * ngroups) / target;
   if (ngroups == 1 && dpad > 0) {
@@ -382,6 +381,22 @@ int pick_R(int64_t ngroups, int64_t ndocs, int dpad, const lik_launch_opts_t* op
     const int64_t wgs = dpad >= 512 ? 250 : dpad >= 256 ? 750 : dpad >= 128 ? 625 : 1250;
     const int64_t r1 = (ndocs + wgs - 1) / wgs;
     if (r1 > R) R = r1;
+  } else if (ngroups > 1 && wg_cu > 0 && dpad > 0 && dpad <= 128) {
+    // Several query blocks: a workgroup costs ~11 us of query-block load and
+    // pipeline fill, as much as 250 doc tokens, so the docs are dealt out in
+    // whole rounds of the chip, one if that leaves at most 48 docs per
+    // workgroup, else rounds of about 32 docs (16 where the lengths vary as
+    // widely as packed corpora's do, so that the last round evens out). k
+    // ranges per XCD: the k * ngroups workgroups there fill its 32 CUs.
+    // Against ~2048 workgroups whatever the size: 256 x 32 query tokens, 256
+    // docs of 50 to 300 tokens 131 -> 93 us (training forward 239 -> 153), 64
+    // queries x 1000 docs 172 -> 96, fp8 64 x 24 tokens x 1000 pages 265 -> 223,
+    // fp32 32 queries x 2048 docs 464 -> 315; 512 x 4096 docs unchanged.
+    const int64_t slots = 32 * wg_cu;
+    const int64_t k = slots > ngroups ? slots / ngroups : 1;
+    const int64_t per = (ndocs + 8 * k - 1) / (8 * k), len = packed ? 16 : 32;
+    const int64_t rounds = per > 48 ? (per + len - 1) / len : 1;
+    R = (ndocs + 8 * k * rounds - 1) / (8 * k * rounds);
   }
   if (opts && opts->docs_per_wg > 0) R = opts->docs_per_wg;  // caller-forced (lik_launch_opts_t)
   if (R < 1) R = 1;
@@ -654,7 +669,8 @@ int maxsim_impl(const lik_seqs_t* Q, const lik_seqs_t* D, uint32_t flags, float 
     if (ps.d.mask) ps.d.mask += j0 * ps.d.msn;
     if (ps.d.lengths) ps.d.lengths += j0;
     if (ps.amax) ps.amax += j0 * ps.amax_ld;
-    ps.R = pick_R(ps.ngroups, n, pl.dpad, opts);
+    const bool two_wg = pl.W == 4 && pl.NSUB >= 4 && !argmax && !(ps.normalize & 2);
+    ps.R = pick_R(ps.ngroups, n, pl.dpad, opts, kd ? 0 : (two_wg ? 2 : 1), D->cu_seqlens != nullptr);
     ps.NR = (n + ps.R - 1) / ps.R;
     ps.xcd_map = ps.NR >= 8 ? 1 : 0;
     const int64_t nb = ps.xcd_map ? ps.ngroups * ((ps.NR + 7) / 8) * 8 : ps.ngroups * ps.NR;
