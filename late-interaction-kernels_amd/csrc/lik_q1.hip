@@ -87,8 +87,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
     const int s = col - ul * p.LU;
     const int64_t u = g * p.QPG + ul;
     bool valid = ul < p.QPG && u < p.nunits;
-    const int64_t q = u / p.nc;
-    const int64_t tok = (u - q * p.nc) * (int64_t)p.LU + s;
+    int64_t q = u / p.nc;
+    int64_t tok = (u - q * p.nc) * (int64_t)p.LU + s;
+    if (p.pair_q) {  // group g is a pair
+      q = p.pair_q[g];
+      tok = p.q_tok0 + s;
+      valid = valid && q >= 0 && q < p.q.n;
+    }
     const char* rowp = nullptr;
     if (valid) {
       valid = tok < seq_len(p.q, q);
@@ -115,11 +120,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
 
   // ---- doc table of this wavefront's range (empty docs score 0 here) ----
   for (int k = lane; k < nloc; k += 64) {
-    const int64_t dg = kd_base + jl0 + k;
+    int64_t dg = kd_base + jl0 + k;
+    if (p.pair_d) {
+      const int64_t pd = p.pair_d[g];
+      dg = pd >= 0 && pd < p.d.n ? pd : -1;  // out of range: scores 0
+    }
     const int64_t L = doc_len<SRC_DENSE>(p, dg);
     const bool skip = p.doc_filter == 1 && p.holes != nullptr && p.holes[dg] != 0;
     s_len[wl][k] = skip ? 0 : (int32_t)L;
-    s_off[wl][k] = p.d.cu ? (int64_t)p.d.cu[dg] * p.d.sl_b : dg * p.d.sn_b;
+    s_off[wl][k] = dg < 0 ? 0 : (p.d.cu ? (int64_t)p.d.cu[dg] * p.d.sl_b : dg * p.d.sn_b);
     if (L == 0 && !skip) {
       for (int t = 0; t < p.QPG; ++t) {
         const int64_t u = g * p.QPG + t;
@@ -414,6 +423,7 @@ int launch_q1_t(const Params& p, bool normq, hipStream_t s) {
 // occupancy) over the launch, at most kQ1RMax; the tile kernel's choice
 // aims at workgroups of several waves and leaves too few wavefronts here.
 int q1_docs_per_wave(const Params& p) {
+  if (p.pair_d) return 1;
   int64_t R = (p.ndocs_pg * p.ngroups + 2047) / 2048;
   R = R < 1 ? 1 : R;
   return (int)(R > kQ1RMax ? kQ1RMax : R);
@@ -422,9 +432,9 @@ int q1_docs_per_wave(const Params& p) {
 // Routed here: 16-bit dense scoring in which one 32-column block holds the
 // columns of a group as planned (W = 1 plans, the KD layout) or of the
 // call's only group (a one-query call whose plan is wider), with nothing in
-// the tile loop beyond the plain max (no doc mask holes, token scales, pair
-// lists or query-chunk accumulation; doc normalisation and argmax at
-// 256-byte rows only), unless the caller forced a column block of several
+// the tile loop beyond the plain max (no doc mask holes, token scales or
+// query-chunk accumulation; doc normalisation and argmax at 256-byte rows
+// only), unless the caller forced a column block of several
 // waves (lik_launch_opts_t). (Two
 // and four blocks per wavefront for queries of up to 128 tokens measured
 // slower than the tile kernel's four waves sharing a tile.)
@@ -433,7 +443,7 @@ bool q1_eligible(int dt, const Plan& pl, const Params& p) {
                          ((int64_t)pl.QPG * pl.LU <= 32) || (pl.ngroups == 1 && pl.nunits * pl.LU <= 32);
   return (dt == LIK_BF16 || dt == LIK_F16) && one_block && pl.dpad >= 64 && pl.dpad <= 512 &&
          ((uintptr_t)p.d.data) % 16 == 0 && p.d.sl_b % 16 == 0 && (p.d.cu || p.d.sn_b % 16 == 0) &&
-         ((!p.amax && !(p.normalize & 2)) || pl.dpad == 128) && !p.pair_q && !p.pair_d && !p.d.mask && !p.d.ts &&
+         ((!p.amax && !(p.normalize & 2)) || pl.dpad == 128) && !p.d.mask && !p.d.ts &&
          !p.q.ts &&
          !p.scale_q && !p.scale_d && p.doc_filter != 2 && !p.accumulate &&
          (int64_t)q1_docs_per_wave(p) * pl.QPG <= kQ1Scores && p.forced_w <= 1;
