@@ -226,7 +226,10 @@ __global__ void __launch_bounds__(W * 64)
     s_dlen[k] = skip ? 0 : ((int32_t)L | (holes ? (int32_t)0x80000000 : 0));
     if (L == 0 && !skip) {
       for (int t = 0; t < p.QPG; ++t)
-        if (float* o = s_outp[t]) ((__attribute__((address_space(1))) float*)o)[k * p.osd] = 0.f;
+        if (float* o = s_outp[t]) {
+          ((__attribute__((address_space(1))) float*)o)[k * p.osd] = 0.f;
+          if ((FEAT & F_ARGMAX) != 0 && p.amax) fill_no_winner(p, unit_of(t), jl);
+        }
     }
   }
   __syncthreads();

@@ -616,9 +616,7 @@ int maxsim_impl(const lik_seqs_t* Q, const lik_seqs_t* D, uint32_t flags, float 
   p.ngroups = pl.ngroups;
   p.kd_K = kd ? D->n / Q->n : 0;
   p.ndocs_pg = kd ? p.kd_K : D->n;
-  if (argmax) {
-    // entries no doc-end reaches (empty docs) stay -1
-    if ((rc = launch_fill_i32(argmax, Q->n * p.ndocs_pg * Q->len, -1, s)) != LIK_OK) return rc;
+  if (argmax) {  // the kernels write every entry, -1 where there is no winner
     p.amax = argmax;
     p.amax_ld = Q->len;
     p.amax_qs = p.ndocs_pg;
@@ -677,6 +675,10 @@ int maxsim_impl(const lik_seqs_t* Q, const lik_seqs_t* D, uint32_t flags, float 
     if (ps.extent) {
       Params p1 = ps;
       p1.d.mask = nullptr;
+      if (q1_eligible(Q->dtype, pl, p1)) {  // one launch takes the docs with holes too
+        p1.doc_filter = 3;
+        return launch_dense(Q->dtype, pl, p1, nb, s);
+      }
       p1.doc_filter = 1;
       int r = launch_dense(Q->dtype, pl, p1, nb, s);
       if (r != LIK_OK) return r;
@@ -735,9 +737,7 @@ int pairs_impl(const lik_seqs_t* Q, const lik_seqs_t* D, const int32_t* pair_q, 
   hipStream_t s = (hipStream_t)stream;
   if (argmax && (Q->dtype == LIK_FP8_E4M3 || Q->token_scale || D->token_scale)) return LIK_ERR_UNSUPPORTED;
   Params p{};
-  if (argmax) {
-    // pairs with no winner stay -1
-    if ((rc = launch_fill_i32(argmax, num_pairs * Q->len, -1, s)) != LIK_OK) return rc;
+  if (argmax) {  // the tile kernels write every entry, -1 where there is no winner
     p.amax = argmax;
     p.amax_ld = Q->len;
     p.amax_qs = 1;
@@ -756,6 +756,7 @@ int pairs_impl(const lik_seqs_t* Q, const lik_seqs_t* D, const int32_t* pair_q, 
     p.ndocs_pg = 1;
     p.nunits = num_pairs;
     p.osq = 1;
+    if (argmax && (rc = launch_fill_i32(argmax, num_pairs * Q->len, -1, s)) != LIK_OK) return rc;
     return launch_maxsim_wide(Q->dtype, p, s);
   }
   Plan pl;

@@ -38,7 +38,9 @@ struct Params {
   const uint8_t* holes;   // per-doc: mask has a False inside [0, extent)
   const uint32_t* tbits;  // per (doc, 32-token tile): row-validity bits of the mask
   int64_t tbits_sn;       // tiles per doc in tbits
-  int doc_filter;         // 0: all docs; 1: docs without mask holes; 2: docs with holes
+  // 0: all docs (no mask); tile kernel: 1 docs without mask holes, 2 docs with
+  // holes; streaming kernel: 3 all docs, those with holes through tbits
+  int doc_filter;
   const int32_t* pair_q;
   const int32_t* pair_d;
   int64_t nunits;  // query units (query x Lq-chunk); pair mode: number of pairs
@@ -95,6 +97,14 @@ __device__ __forceinline__ int64_t doc_len(const Params& p, int64_t j) {
     if (p.extent) return p.extent[j];
     return seq_len(p.d, j);
   }
+}
+
+// argmax row of unit u and doc jl of its group: "no winner" (an empty doc).
+__device__ __forceinline__ void fill_no_winner(const Params& p, int64_t u, int64_t jl) {
+  const int64_t q = u / p.nc;
+  const int64_t t0 = p.q_tok0 + (u - q * p.nc) * p.LU;
+  int32_t* row = p.amax + (q * p.amax_qs + jl) * p.amax_ld;
+  for (int64_t t = t0; t < t0 + p.LU && t < p.amax_ld; ++t) row[t] = -1;
 }
 
 // Config legality: B-fragment registers per lane must stay <= 128 VGPRs.

@@ -44,7 +44,7 @@ constexpr int kQ1Scores = 256;  // doc scores per wavefront held until the loop 
 // kernel does it (a row's 16 chunk sums of squares added as a balanced tree
 // in chunk order: each lane holds chunks 0..7 or 8..15 of its row, the two
 // halves meet by one lane swap; scaled in fp32 and rounded once).
-template <int EK, int DPAD, bool FULLD, bool NORMQ, bool EXT = false>
+template <int EK, int DPAD, bool FULLD, bool NORMQ, bool EXT, bool HOLES>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) maxsim_q1_kernel(const Params p) {
   using T = KT<EK, DPAD>;
   constexpr int KS = T::KSTEPS;
@@ -126,13 +126,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
       dg = pd >= 0 && pd < p.d.n ? pd : -1;  // out of range: scores 0
     }
     const int64_t L = doc_len<SRC_DENSE>(p, dg);
-    const bool skip = p.doc_filter == 1 && p.holes != nullptr && p.holes[dg] != 0;
-    s_len[wl][k] = skip ? 0 : (int32_t)L;
+    const bool holed = HOLES && p.holes[dg] != 0;
+    s_len[wl][k] = (int32_t)L | (holed ? (int32_t)0x80000000 : 0);
     s_off[wl][k] = dg < 0 ? 0 : (p.d.cu ? (int64_t)p.d.cu[dg] * p.d.sl_b : dg * p.d.sn_b);
-    if (L == 0 && !skip) {
+    if (L == 0) {
       for (int t = 0; t < p.QPG; ++t) {
         const int64_t u = g * p.QPG + t;
-        if (u < p.nunits) p.out[u * p.osq + (jl0 + k) * p.osd] = 0.f;
+        if (u >= p.nunits) break;
+        p.out[u * p.osq + (jl0 + k) * p.osd] = 0.f;
+        if (EXT && p.amax) fill_no_winner(p, u, jl0 + k);
       }
     }
   }
@@ -166,13 +168,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
   // ---- cursor: unit c of tile t of local doc k (k == nloc: past the range) ----
   struct Cur {
     int k, t, len;
+    bool holes;
     int64_t off;
   };
   auto cur_doc = [&](Cur& c, int k) {
     while (k < nloc && s_len[wl][k] == 0) ++k;
     c.k = k;
     c.t = 0;
-    c.len = k < nloc ? __builtin_amdgcn_readfirstlane(s_len[wl][k]) : 0;
+    const int v = k < nloc ? __builtin_amdgcn_readfirstlane(s_len[wl][k]) : 0;
+    c.len = HOLES ? v & 0x7fffffff : v;
+    c.holes = HOLES && v < 0;
     const int64_t o = k < nloc ? s_off[wl][k] : 0;
     c.off = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)o) |
             ((int64_t)__builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)o >> 32)) << 32);
@@ -180,6 +185,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
   struct Desc {
     int nv, k, t;  // valid rows, local doc, tile of the doc
     bool docend;   // last unit of the doc's last tile
+    bool holes;    // the doc's mask drops tokens before its last kept one
   };
   // DMA of unit CU of the cursor's tile into ring slot S (exactly NI load
   // instructions, whether or not the tile exists); after the tile's last
@@ -191,6 +197,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
     d.nv = rem < 32 ? rem : 32;
     d.k = c.k;
     d.t = c.t;
+    d.holes = c.holes;
     const bool tile_end = c.len > 0 && rem <= 32;
     d.docend = tile_end && CU == NU - 1;
     // the buffer covers rows [32 t, len) of the doc: later rows read 0
@@ -313,6 +320,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
           }
       }
     }
+    // Docs whose mask has holes (a uniform branch): the tile's validity word,
+    // by a scalar load (the loop's only vector loads are the counted DMAs).
+    // Dropped rows are zeroed before their MFMAs (a NaN there must not reach
+    // the max) and set to -inf after.
+    uint32_t vb = 0xffffffffu;
+    if (HOLES && d.holes) {
+      typedef __attribute__((address_space(4))) const uint32_t* cptr;
+      vb = ((cptr)(uintptr_t)(p.tbits + (kd_base + jl0 + d.k) * p.tbits_sn))[d.t];
+      const bool keep = (vb >> l32) & 1u;
+#pragma unroll
+      for (int ks = 0; ks < KSU; ++ks) af[ks] = keep ? af[ks] : u32x4{0u, 0u, 0u, 0u};
+    }
 #pragma unroll
     for (int ks = 0; ks < KSU; ++ks)
       acc = mfma32<EK>(CU == 0 && ks == 0 ? f32x16{} : acc, &af[ks], &bq[CU * KSU + ks]);
@@ -323,6 +342,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
 #pragma unroll
         for (int e = 0; e < 16; ++e)
           if (8 * (e >> 2) + (e & 3) >= lim) acc[e] = NEG_INF;
+      }
+      if (HOLES && d.holes) {
+        const uint32_t vh = vb >> (4 * h);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[e] = ((vh >> (8 * (e >> 2) + (e & 3))) & 1u) ? acc[e] : NEG_INF;
       }
       if (EXT && p.amax) {
         // rows in increasing order; only a strictly larger value replaces
@@ -382,41 +406,36 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
   for (int i = lane; i < nloc * p.QPG; i += 64) {
     const int k = i / p.QPG, t = i - k * p.QPG;
     const int64_t u = g * p.QPG + t;
-    if (u < p.nunits && s_len[wl][k] > 0) p.out[u * p.osq + (jl0 + k) * p.osd] = s_score[wl][i];
+    if (u < p.nunits && s_len[wl][k] != 0) p.out[u * p.osq + (jl0 + k) * p.osd] = s_score[wl][i];
   }
 }
 
-template <int EK, int DPAD>
-int launch_q1_t(const Params& p, bool normq, hipStream_t s) {
-  if constexpr (DPAD == 128) {
-    if (p.amax || (p.normalize & 2)) {
-      const int64_t waves = p.ngroups * p.NR;
-      const int64_t nb = (waves + 3) / 4;
-      if (nb <= 0) return LIK_OK;
-      if (nb > 0x7fffffffLL) return LIK_ERR_UNSUPPORTED;
-      auto go = [&](auto kern) {
-        launch_kernel(kern, dim3((unsigned)nb), dim3(256), 0, s, p);
-        return hipGetLastError() == hipSuccess ? LIK_OK : LIK_ERR_LAUNCH;
-      };
-      const bool full = p.d.dim == DPAD && p.q.dim == DPAD;
-      if (full)
-        return normq ? go(maxsim_q1_kernel<EK, DPAD, true, true, true>) : go(maxsim_q1_kernel<EK, DPAD, true, false, true>);
-      return normq ? go(maxsim_q1_kernel<EK, DPAD, false, true, true>) : go(maxsim_q1_kernel<EK, DPAD, false, false, true>);
-    }
-  }
-  if (p.amax || (p.normalize & 2)) return LIK_ERR_UNSUPPORTED;
+template <int EK, int DPAD, bool EXT, bool HOLES>
+int launch_q1_f(const Params& p, bool normq, hipStream_t s) {
   const int64_t waves = p.ngroups * p.NR;
   const int64_t nb = (waves + 3) / 4;
   if (nb <= 0) return LIK_OK;
   if (nb > 0x7fffffffLL) return LIK_ERR_UNSUPPORTED;
-  const bool full = p.d.dim == DPAD && p.q.dim == DPAD;
   auto go = [&](auto kern) {
     launch_kernel(kern, dim3((unsigned)nb), dim3(256), 0, s, p);
     return hipGetLastError() == hipSuccess ? LIK_OK : LIK_ERR_LAUNCH;
   };
-  if (full)
-    return normq ? go(maxsim_q1_kernel<EK, DPAD, true, true>) : go(maxsim_q1_kernel<EK, DPAD, true, false>);
-  return normq ? go(maxsim_q1_kernel<EK, DPAD, false, true>) : go(maxsim_q1_kernel<EK, DPAD, false, false>);
+  if (p.d.dim == DPAD && p.q.dim == DPAD)
+    return normq ? go(maxsim_q1_kernel<EK, DPAD, true, true, EXT, HOLES>)
+                 : go(maxsim_q1_kernel<EK, DPAD, true, false, EXT, HOLES>);
+  return normq ? go(maxsim_q1_kernel<EK, DPAD, false, true, EXT, HOLES>)
+               : go(maxsim_q1_kernel<EK, DPAD, false, false, EXT, HOLES>);
+}
+
+template <int EK, int DPAD>
+int launch_q1_t(const Params& p, bool normq, hipStream_t s) {
+  const bool holes = p.doc_filter == 3;
+  if (p.amax || (p.normalize & 2)) {
+    if constexpr (DPAD == 128)
+      return holes ? launch_q1_f<EK, DPAD, true, true>(p, normq, s) : launch_q1_f<EK, DPAD, true, false>(p, normq, s);
+    return LIK_ERR_UNSUPPORTED;
+  }
+  return holes ? launch_q1_f<EK, DPAD, false, true>(p, normq, s) : launch_q1_f<EK, DPAD, false, false>(p, normq, s);
 }
 
 // Docs per wavefront: about 2048 wavefronts (two per SIMD, the kernel's
@@ -432,9 +451,9 @@ int q1_docs_per_wave(const Params& p) {
 // Routed here: 16-bit dense scoring in which one 32-column block holds the
 // columns of a group as planned (W = 1 plans, the KD layout) or of the
 // call's only group (a one-query call whose plan is wider), with nothing in
-// the tile loop beyond the plain max (no doc mask holes, token scales or
-// query-chunk accumulation; doc normalisation and argmax at 256-byte rows
-// only), unless the caller forced a column block of several
+// the tile loop beyond the plain max (no token scales or query-chunk
+// accumulation; doc normalisation and argmax at 256-byte rows only; masks come
+// as the pre-pass's summary, docs with holes included), unless the caller forced a column block of several
 // waves (lik_launch_opts_t). (Two
 // and four blocks per wavefront for queries of up to 128 tokens measured
 // slower than the tile kernel's four waves sharing a tile.)

@@ -137,12 +137,12 @@ def dense_maxsim_train(
     Nd, Ld, _ = D.shape
     docs = (Nd // Nq if Nq else 0) if kd else Nd
     out = torch.empty(Nq, docs, device=Q.device, dtype=torch.float32)
-    argmax = torch.full((Nq * docs, Lq), -1, device=Q.device, dtype=torch.int32)
+    argmax = torch.empty((Nq * docs, Lq), device=Q.device, dtype=torch.int32)  # every entry is written
     Qp = _lib.prepare_tokens(Q.detach())
     Dp = _lib.prepare_tokens(D.detach())
     qm = _mask_i8(q_mask, (Nq, Lq))
     if Nq == 0 or docs == 0 or Lq == 0 or Ld == 0:
-        return out.zero_(), argmax, Qp, Dp, qm
+        return out.zero_(), argmax.fill_(-1), Qp, Dp, qm
     dm = _mask_i8(d_mask, (Nd, Ld))
     qs = _lib.seqs(Qp, n=Nq, length=Lq, stride_n=Qp.stride(0), stride_l=Qp.stride(1), mask=qm,
                    mask_strides=(qm.stride(0), qm.stride(1)) if qm is not None else (0, 0))
@@ -228,12 +228,12 @@ def packed_maxsim_train(Q_packed, D_packed, cu_q, cu_d, max_q: int, max_d: int):
     _lib.require_gpu(Q_packed, D_packed, cu_q, cu_d)
     Nq = cu_q.numel() - 1
     Nd = cu_d.numel() - 1
-    out = torch.zeros(max(Nq, 0), max(Nd, 0), device=Q_packed.device, dtype=torch.float32)
-    argmax = torch.full((max(Nq, 0) * max(Nd, 0), max(max_q, 0)), -1, device=Q_packed.device, dtype=torch.int32)
+    out = torch.empty(max(Nq, 0), max(Nd, 0), device=Q_packed.device, dtype=torch.float32)
+    argmax = torch.empty((max(Nq, 0) * max(Nd, 0), max(max_q, 0)), device=Q_packed.device, dtype=torch.int32)
     Qp = _lib.prepare_tokens(Q_packed.detach())
     Dp = _lib.prepare_tokens(D_packed.detach())
     if Nq <= 0 or Nd <= 0 or max_q <= 0 or Q_packed.shape[0] == 0 or D_packed.shape[0] == 0:
-        return out, argmax, Qp, Dp
+        return out.zero_(), argmax.fill_(-1), Qp, Dp
     qs = _lib.seqs(Qp, n=Nq, length=max_q, stride_l=Qp.stride(0), cu=cu_q)
     ds = _lib.seqs(Dp, n=Nd, length=max(int(max_d), 0), stride_l=Dp.stride(0), cu=cu_d)
     lib = _lib.load()
@@ -318,12 +318,12 @@ def pairs_maxsim_train(Q_packed, D_packed, cu_q, cu_d, pair_q, pair_d, max_q: in
     """Pair-list training forward: ``(scores [P], argmax [P, max_q], Qp, Dp)``."""
     _lib.require_gpu(Q_packed, D_packed, cu_q, cu_d, pair_q, pair_d)
     P = pair_q.numel()
-    out = torch.zeros(P, device=Q_packed.device, dtype=torch.float32)
-    argmax = torch.full((P, max(max_q, 0)), -1, device=Q_packed.device, dtype=torch.int32)
+    out = torch.empty(P, device=Q_packed.device, dtype=torch.float32)
+    argmax = torch.empty((P, max(max_q, 0)), device=Q_packed.device, dtype=torch.int32)
     Qp = _lib.prepare_tokens(Q_packed.detach())
     Dp = _lib.prepare_tokens(D_packed.detach())
     if P == 0 or max_q <= 0 or Q_packed.shape[0] == 0 or D_packed.shape[0] == 0:
-        return out, argmax, Qp, Dp
+        return out.zero_(), argmax.fill_(-1), Qp, Dp
     qs = _lib.seqs(Qp, n=cu_q.numel() - 1, length=max_q, stride_l=Qp.stride(0), cu=cu_q)
     ds = _lib.seqs(Dp, n=cu_d.numel() - 1, length=max(int(max_d), 0), stride_l=Dp.stride(0), cu=cu_d)
     lib = _lib.load()

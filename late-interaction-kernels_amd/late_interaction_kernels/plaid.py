@@ -338,7 +338,7 @@ class _ResidualQGradFn(torch.autograd.Function):
             ds = _lib.seqs(dec, n=Nd, length=L, stride_n=L * dec.stride(0), stride_l=dec.stride(0), lengths=lengths)
         flags = _lib.LIK_NORMALIZE_Q if normalize else 0
         out = torch.empty(Nq, Nd, device=Q.device, dtype=torch.float32)
-        argmax = torch.full((Nq * Nd, Lq), -1, device=Q.device, dtype=torch.int32)
+        argmax = torch.empty((Nq * Nd, Lq), device=Q.device, dtype=torch.int32)  # every entry is written
         lib = _lib.load()
         nbytes = lib.lik_maxsim_workspace_size(ctypes.byref(qs), ctypes.byref(ds), flags)
         ws = _lib.workspace(nbytes, Q.device)
