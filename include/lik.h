@@ -404,6 +404,24 @@ int lik_topk_select(const float* scores, int64_t rows, int64_t n, int64_t ld, in
                     int64_t out_ld, void* workspace, size_t workspace_bytes, lik_stream_t stream);
 
 /*
+ * Projection-head gradients of maxsim_from_hidden training: from grad_d
+ * [H->n * H->len, dp] (lik_maxsim_backward's grad_D, 16-byte aligned, zero past
+ * d_out) and the forward's argmax [nq * H->n, lq],
+ *   grad_h [n * len, dim] = grad_d W on the rows that won a max, else zeros
+ *   grad_w [d_out, dim] = sum over those rows of grad_d^T H, grad_b = sum of grad_d
+ * H: bf16 / fp16, padded, last dim contiguous, dim a multiple of 8, len <=
+ * 65536; W [d_out, dim] (16-byte rows, row stride w_stride elements) and grad_h / grad_w in
+ * H's dtype, grad_b fp32; dp a multiple of 8, <= 128. A null output is skipped.
+ * Replaces fused_head.py:347-460. The workspace size is 0 for shapes not taken
+ * (LIK_ERR_UNSUPPORTED).
+ */
+size_t lik_head_backward_workspace_size(int32_t dtype, int64_t nq, int64_t lq, int64_t nd, int64_t ld, int64_t dp,
+                                        int64_t d_out, int64_t d_model);
+int lik_head_backward(const int32_t* argmax, int64_t nq, int64_t lq, const void* grad_d, int64_t dp,
+                      const lik_seqs_t* H, const void* W, int64_t w_stride, int64_t d_out, void* grad_h, void* grad_w,
+                      float* grad_b, void* workspace, size_t workspace_bytes, lik_stream_t stream);
+
+/*
  * fp8 (OCP e4m3fn) quantisation of x [rows, dim] (contiguous, bf16 / fp16 /
  * fp32): scale = max(amax, 1e-6) / 448 in fp32, out = e4m3(clamp(x / scale)),
  * round to nearest even. With LIK_PER_TOKEN scale is [rows], else one value.

@@ -415,3 +415,34 @@ def from_hidden_forward(Q, H, W, b, d_mask, *, normalize: bool, want_argmax: boo
     _lib.check(rc, "lik_maxsim_from_hidden")
     return out, argmax
 
+
+
+def head_backward(argmax, Nq: int, Lq: int, gd, H, W, *, need_h: bool, need_w: bool, need_b: bool):
+    """Projection-head gradients (``lik_head_backward``): ``(grad_H, grad_W, grad_b fp32)``
+    with ``None`` where not needed, or ``None`` for calls the kernels do not take
+    (fp32, mixed dtypes, d_out > 128, d_model % 8, docs of more than 65536 tokens)."""
+    Nd, Ld, d_model = H.shape
+    dp, d_out = gd.shape[-1], W.shape[0]
+    if not (H.dtype == W.dtype == gd.dtype and H.dtype in (torch.bfloat16, torch.float16)) or not _lib.plain_op(gd, H, W):
+        return None
+    lib = _lib.load()
+    nbytes = lib.lik_head_backward_workspace_size(_lib.DTYPE_CODE[H.dtype], Nq, Lq, Nd, Ld, dp, d_out, d_model)
+    if nbytes == 0 or gd.data_ptr() % 16:
+        return None
+    if H.stride(-1) != 1 or H.data_ptr() % 4 or any(s % 2 for s in H.stride()[:-1]):
+        H = H.contiguous()
+    if W.stride(-1) != 1 or W.data_ptr() % 16 or W.stride(0) % 8:
+        W = W.contiguous()
+    gh = torch.empty(H.shape, dtype=H.dtype, device=H.device) if need_h else None
+    gw = torch.empty(W.shape, dtype=W.dtype, device=W.device) if need_w else None
+    gb = torch.empty(d_out, dtype=torch.float32, device=W.device) if need_b else None
+    hs = _lib.seqs(H, n=Nd, length=Ld, stride_n=H.stride(0), stride_l=H.stride(1))
+    ws = _lib.workspace(nbytes, H.device)
+    with torch.cuda.device(H.device):
+        rc = lib.lik_head_backward(argmax.data_ptr(), Nq, Lq, gd.data_ptr(), dp, ctypes.byref(hs), W.data_ptr(),
+                                   W.stride(0), d_out, _lib.ptr(gh), _lib.ptr(gw), _lib.ptr(gb), _lib.ptr(ws), nbytes,
+                                   _lib.stream_of(gd))
+    if rc == _lib.LIK_ERR_UNSUPPORTED:
+        return None
+    _lib.check(rc, "lik_head_backward")
+    return gh, gw, gb

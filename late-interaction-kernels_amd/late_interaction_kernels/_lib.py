@@ -74,6 +74,8 @@ EXPORTED_SYMBOLS = (
     "lik_plaid_token_records",
     "lik_plaid_maxsim_qc",
     "lik_plaid_maxsim_qc_workspace_size",
+    "lik_head_backward",
+    "lik_head_backward_workspace_size",
     "lik_quantize_fp8",
     "lik_quantize_fp8_workspace_size",
 )
@@ -225,6 +227,11 @@ def load() -> ctypes.CDLL:
     lib.lik_plaid_maxsim_qc.argtypes = [P(LikSeqs), P(LikPlaidDocs), _p, ctypes.c_uint32, _p, _i64, _i64, _p,
                                         ctypes.c_size_t, P(LikLaunchOpts), _p]
     lib.lik_plaid_maxsim_qc.restype = ctypes.c_int
+    lib.lik_head_backward_workspace_size.argtypes = [_i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64]
+    lib.lik_head_backward_workspace_size.restype = ctypes.c_size_t
+    lib.lik_head_backward.argtypes = [_p, _i64, _i64, _p, _i64, P(LikSeqs), _p, _i64, _i64, _p, _p, _p, _p,
+                                      ctypes.c_size_t, _p]
+    lib.lik_head_backward.restype = ctypes.c_int
     lib.lik_quantize_fp8_workspace_size.argtypes = [ctypes.c_uint32]
     lib.lik_quantize_fp8_workspace_size.restype = ctypes.c_size_t
     lib.lik_quantize_fp8.argtypes = [_p, _i32, _i64, _i32, ctypes.c_uint32, _p, _p, _p, ctypes.c_size_t, _p]

@@ -14,8 +14,9 @@ tokens) project with one GEMM (``F.linear``) and score the materialised docs.
 Training: the projection is one GEMM, then the argmax-saving MaxSim kernel
 with the doc-only normalise. Only doc tokens that won some query token's max
 have a gradient, so the projection's gradients are taken on those rows alone:
-grad_W = g^T H_win, grad_b = sum g and grad_H = g W scattered into a zeroed
-tensor (the reference's backward, fused_head.py:347-460, gathers H at the
+grad_W = g^T H_win, grad_b = sum g and grad_H = g W on those rows, zeros
+elsewhere (``lik_head_backward``; by torch operators for shapes and dtypes it
+does not take; the reference's backward, fused_head.py:347-460, gathers H at the
 winners the same way). Projecting first is the faster training route here:
 with the fused forward, the backward has to gather and project the winning
 rows again, and those extra small launches cost more than the fused forward
@@ -33,7 +34,7 @@ from __future__ import annotations
 import torch
 
 from .autograd import _needs_grad, _score, _validate_devices
-from ._core import dense_maxsim_train, from_hidden_forward, maxsim_backward, unify_dtype
+from ._core import dense_maxsim_train, from_hidden_forward, head_backward, maxsim_backward, unify_dtype
 
 
 class _FromHiddenFn(torch.autograd.Function):
@@ -59,6 +60,13 @@ class _FromHiddenFn(torch.autograd.Function):
         Nq, Lq, d_out = Qp.shape[0], Qp.shape[1], W.shape[0]
         Nd, Ld, d_model = H_d.shape
         grad_q = gq[..., :d_out].to(ctx.q_dtype) if ctx.needs_input_grad[0] else None
+        need_b = ctx.has_b and ctx.needs_input_grad[3]
+        done = head_backward(argmax, Nq, Lq, gd, H_d, W, need_h=ctx.needs_input_grad[1],
+                             need_w=ctx.needs_input_grad[2], need_b=need_b)
+        if done is not None:
+            grad_h, grad_w, grad_b = done
+            return grad_q, grad_h, grad_w, None if grad_b is None else grad_b.to(ctx.b_dtype), None, None
+        # other dtypes and shapes, by operators:
         # doc rows that won a max (the only rows with a nonzero grad_D)
         am = argmax.view(Nq, Nd, Lq)
         rows = (torch.arange(Nd, device=am.device).view(1, Nd, 1) * Ld + am.long())[am >= 0]
