@@ -404,6 +404,15 @@ int lik_topk_select(const float* scores, int64_t rows, int64_t n, int64_t ld, in
                     int64_t out_ld, void* workspace, size_t workspace_bytes, lik_stream_t stream);
 
 /*
+ * *ok = 1 if every sequence of cu_a [n_a + 1] is at most max_a long and every one
+ * of cu_b [n_b + 1] at most max_b, else 0 (the caller-supplied max_seqlen
+ * bounds, _utils.py:32-50; the arrays may be the same). One workgroup: for at
+ * most some ten thousand sequences.
+ */
+int lik_seqlens_cover(const int32_t* cu_a, int64_t n_a, int64_t max_a, const int32_t* cu_b, int64_t n_b, int64_t max_b,
+                      uint8_t* ok, lik_stream_t stream);
+
+/*
  * Projection-head gradients of maxsim_from_hidden training: from grad_d
  * [H->n * H->len, dp] (lik_maxsim_backward's grad_D, 16-byte aligned, zero past
  * d_out) and the forward's argmax [nq * H->n, lq],

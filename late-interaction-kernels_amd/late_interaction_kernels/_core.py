@@ -152,7 +152,7 @@ def dense_maxsim_train(
     lib = _lib.load()
     nbytes = lib.lik_maxsim_workspace_size(ctypes.byref(qs), ctypes.byref(ds), flags)
     ws = _lib.workspace(nbytes, Q.device)
-    with torch.cuda.device(Q.device):
+    with _lib.on_device(Q.device):
         rc = lib.lik_maxsim_argmax(ctypes.byref(qs), ctypes.byref(ds), flags, out.data_ptr(), out.stride(0),
                                    out.stride(1), argmax.data_ptr(), _lib.ptr(ws), nbytes, _lib.stream_of(out))
     _lib.check(rc, "lik_maxsim_argmax")
@@ -184,7 +184,7 @@ def maxsim_backward(
     lib = _lib.load()
     nbytes = lib.lik_maxsim_backward_workspace_size(ctypes.byref(qs), ctypes.byref(ds), flags)
     ws = _lib.workspace(nbytes, Qp.device)
-    with torch.cuda.device(Qp.device):
+    with _lib.on_device(Qp.device):
         rc = lib.lik_maxsim_backward(g.data_ptr(), g.stride(0), ctypes.byref(qs), ctypes.byref(ds), argmax.data_ptr(),
                                      flags, gq.data_ptr(), gd.data_ptr(), _lib.ptr(ws), nbytes,
                                      _lib.stream_of(gq))
@@ -239,7 +239,7 @@ def packed_maxsim_train(Q_packed, D_packed, cu_q, cu_d, max_q: int, max_d: int):
     lib = _lib.load()
     nbytes = lib.lik_maxsim_workspace_size(ctypes.byref(qs), ctypes.byref(ds), 0)
     ws = _lib.workspace(nbytes, Q_packed.device)
-    with torch.cuda.device(Q_packed.device):
+    with _lib.on_device(Q_packed.device):
         rc = lib.lik_maxsim_argmax(ctypes.byref(qs), ctypes.byref(ds), 0, out.data_ptr(), out.stride(0),
                                    out.stride(1), argmax.data_ptr(), _lib.ptr(ws), nbytes, _lib.stream_of(out))
     _lib.check(rc, "lik_maxsim_argmax")
@@ -261,7 +261,7 @@ def packed_backward(grad, Qp, Dp, cu_q, cu_d, argmax, max_q: int, max_d: int, *,
     lib = _lib.load()
     nbytes = lib.lik_maxsim_backward_workspace_size(ctypes.byref(qs), ctypes.byref(ds), 0)
     ws = _lib.workspace(nbytes, Qp.device)
-    with torch.cuda.device(Qp.device):
+    with _lib.on_device(Qp.device):
         rc = lib.lik_maxsim_backward(g.data_ptr(), g.stride(0), ctypes.byref(qs), ctypes.byref(ds), argmax.data_ptr(),
                                      0, gq.data_ptr(), _lib.ptr(gd), _lib.ptr(ws), nbytes, _lib.stream_of(gq))
     _lib.check(rc, "lik_maxsim_backward")
@@ -273,7 +273,7 @@ def _launch(qs, ds, flags: int, out_scale: float, out: torch.Tensor, device: tor
     opts = _lib.call_opts()
     nbytes = lib.lik_maxsim_workspace_size_ex(ctypes.byref(qs), ctypes.byref(ds), flags, opts)
     ws = _lib.workspace(nbytes, device)
-    with torch.cuda.device(device):
+    with _lib.on_device(device):
         rc = lib.lik_maxsim_ex(
             ctypes.byref(qs), ctypes.byref(ds), flags, float(out_scale), out.data_ptr(), out.stride(0),
             out.stride(1), _lib.ptr(ws), nbytes, opts, _lib.stream_of(out),
@@ -305,7 +305,7 @@ def pairs_maxsim(
     qs = _lib.seqs(Qp, n=cq.numel() - 1, length=max_q, stride_l=Qp.stride(0), cu=cq)
     ds = _lib.seqs(Dp, n=cd.numel() - 1, length=max(int(max_d), 0), stride_l=Dp.stride(0), cu=cd)
     lib = _lib.load()
-    with torch.cuda.device(Q_packed.device):
+    with _lib.on_device(Q_packed.device):
         rc = lib.lik_maxsim_pairs(
             ctypes.byref(qs), ctypes.byref(ds), pq.data_ptr(), pd.data_ptr(), P, 0, out.data_ptr(),
             _lib.stream_of(out),
@@ -327,7 +327,7 @@ def pairs_maxsim_train(Q_packed, D_packed, cu_q, cu_d, pair_q, pair_d, max_q: in
     qs = _lib.seqs(Qp, n=cu_q.numel() - 1, length=max_q, stride_l=Qp.stride(0), cu=cu_q)
     ds = _lib.seqs(Dp, n=cu_d.numel() - 1, length=max(int(max_d), 0), stride_l=Dp.stride(0), cu=cu_d)
     lib = _lib.load()
-    with torch.cuda.device(Q_packed.device):
+    with _lib.on_device(Q_packed.device):
         rc = lib.lik_maxsim_pairs_argmax(ctypes.byref(qs), ctypes.byref(ds), pair_q.data_ptr(), pair_d.data_ptr(), P,
                                          0, out.data_ptr(), argmax.data_ptr(), _lib.stream_of(out))
     _lib.check(rc, "lik_maxsim_pairs_argmax")
@@ -348,7 +348,7 @@ def pairs_backward(grad, Qp, Dp, cu_q, cu_d, pair_q, pair_d, argmax, max_q: int,
     lib = _lib.load()
     nbytes = lib.lik_maxsim_pairs_backward_workspace_size(ctypes.byref(qs), ctypes.byref(ds), P)
     ws = _lib.workspace(nbytes, Qp.device)
-    with torch.cuda.device(Qp.device):
+    with _lib.on_device(Qp.device):
         rc = lib.lik_maxsim_pairs_backward(g.data_ptr(), ctypes.byref(qs), ctypes.byref(ds), pair_q.data_ptr(),
                                            pair_d.data_ptr(), P, argmax.data_ptr(), 0, gq.data_ptr(), _lib.ptr(gd),
                                            _lib.ptr(ws), nbytes, _lib.stream_of(gq))
@@ -363,17 +363,38 @@ def seqlen_max(cu: torch.Tensor) -> int:
     return int((cu[1:] - cu[:-1]).max().item())
 
 
-def assert_max_seqlen_covers(cu: torch.Tensor, max_seqlen: int, name: str) -> None:
-    """On-device check that a caller-supplied bound covers every sequence
-    (``_utils.py:32-50``): the bound sizes the query block, so a too-small
-    value would drop tokens."""
-    if cu.numel() <= 1:
+_COVER_MAX = 1 << 15  # sequences the one-workgroup check reads (more: torch's reductions)
+
+
+def assert_max_seqlens_cover(*checks: tuple[torch.Tensor, int | None, str]) -> None:
+    """On-device check that caller-supplied bounds cover every sequence of one or
+    two ``cu_seqlens`` (``_utils.py:32-50``): a bound sizes the query block, so a
+    too-small value would drop tokens. One kernel reads both arrays
+    (``lik_seqlens_cover``); the differences, maximum and comparison as torch
+    operators are three launches for each."""
+    todo = [(cu, m, name) for cu, m, name in checks if m is not None and cu.numel() > 1]
+    if not todo:
         return
-    torch._assert_async(
-        (cu[1:] - cu[:-1]).max().le(max_seqlen),
-        f"{name}={max_seqlen} is smaller than the longest sequence in cu_seqlens; "
-        "it is a hard bound and would silently truncate tokens.",
-    )
+    if (len(todo) <= 2 and sum(cu.numel() for cu, _, _ in todo) <= _COVER_MAX
+            and all(cu.device == todo[0][0].device and cu.dtype == torch.int32 and cu.is_contiguous()
+                    and abs(m) < 1 << 62 for cu, m, _ in todo)
+            and _lib.plain_op(*(cu for cu, _, _ in todo))):
+        ok = torch.empty((), device=todo[0][0].device, dtype=torch.bool)
+        (a, ma, _), (b, mb, _) = todo[0], todo[-1]
+        with _lib.on_device(ok.device):
+            rc = _lib.load().lik_seqlens_cover(a.data_ptr(), a.numel() - 1, ma, b.data_ptr(), b.numel() - 1, mb,
+                                               ok.data_ptr(), _lib.stream_of(ok))
+        _lib.check(rc, "lik_seqlens_cover")
+        names = " or ".join(f"{name}={m}" for _, m, name in todo)
+        torch._assert_async(ok, f"{names} is smaller than the longest sequence in cu_seqlens; "
+                            "it is a hard bound and would silently truncate tokens.")
+        return
+    for cu, m, name in todo:
+        torch._assert_async(
+            (cu[1:] - cu[:-1]).max().le(m),
+            f"{name}={m} is smaller than the longest sequence in cu_seqlens; "
+            "it is a hard bound and would silently truncate tokens.",
+        )
 
 
 def from_hidden_forward(Q, H, W, b, d_mask, *, normalize: bool, want_argmax: bool):
@@ -406,7 +427,7 @@ def from_hidden_forward(Q, H, W, b, d_mask, *, normalize: bool, want_argmax: boo
     nbytes = lib.lik_maxsim_from_hidden_workspace_size(ctypes.byref(qs), ctypes.byref(hs))
     ws = _lib.workspace(nbytes, Q.device)
     flags = (_lib.LIK_NORMALIZE_D if normalize else 0) | (_lib.LIK_BIAS_16 if bias16 else 0)
-    with torch.cuda.device(Q.device):
+    with _lib.on_device(Q.device):
         rc = lib.lik_maxsim_from_hidden(ctypes.byref(qs), ctypes.byref(hs), Wc.data_ptr(), Wc.stride(0),
                                         _lib.ptr(bias), flags, out.data_ptr(), out.stride(0), out.stride(1),
                                         _lib.ptr(argmax), _lib.ptr(ws), nbytes, _lib.stream_of(out))
@@ -438,7 +459,7 @@ def head_backward(argmax, Nq: int, Lq: int, gd, H, W, *, need_h: bool, need_w: b
     gb = torch.empty(d_out, dtype=torch.float32, device=W.device) if need_b else None
     hs = _lib.seqs(H, n=Nd, length=Ld, stride_n=H.stride(0), stride_l=H.stride(1))
     ws = _lib.workspace(nbytes, H.device)
-    with torch.cuda.device(H.device):
+    with _lib.on_device(H.device):
         rc = lib.lik_head_backward(argmax.data_ptr(), Nq, Lq, gd.data_ptr(), dp, ctypes.byref(hs), W.data_ptr(),
                                    W.stride(0), d_out, _lib.ptr(gh), _lib.ptr(gw), _lib.ptr(gb), _lib.ptr(ws), nbytes,
                                    _lib.stream_of(gd))

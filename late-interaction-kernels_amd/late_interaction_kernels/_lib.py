@@ -78,6 +78,7 @@ EXPORTED_SYMBOLS = (
     "lik_head_backward_workspace_size",
     "lik_quantize_fp8",
     "lik_quantize_fp8_workspace_size",
+    "lik_seqlens_cover",
 )
 
 _p = ctypes.c_void_p
@@ -232,6 +233,8 @@ def load() -> ctypes.CDLL:
     lib.lik_head_backward.argtypes = [_p, _i64, _i64, _p, _i64, P(LikSeqs), _p, _i64, _i64, _p, _p, _p, _p,
                                       ctypes.c_size_t, _p]
     lib.lik_head_backward.restype = ctypes.c_int
+    lib.lik_seqlens_cover.argtypes = [_p, _i64, _i64, _p, _i64, _i64, _p, _p]
+    lib.lik_seqlens_cover.restype = ctypes.c_int
     lib.lik_quantize_fp8_workspace_size.argtypes = [ctypes.c_uint32]
     lib.lik_quantize_fp8_workspace_size.restype = ctypes.c_size_t
     lib.lik_quantize_fp8.argtypes = [_p, _i32, _i64, _i32, ctypes.c_uint32, _p, _p, _p, ctypes.c_size_t, _p]
@@ -272,7 +275,25 @@ def plain_op(*tensors: torch.Tensor) -> bool:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
+
+
+class _Here:
+    """A context that changes nothing."""
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return None
+
+
+_HERE = _Here()
+
+
+def on_device(device: torch.device):
+    """``torch.cuda.device(device)``, or nothing when that device is the current one."""
+    return _HERE if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
@@ -302,21 +323,12 @@ def seqs(
     token_scale: torch.Tensor | None = None,
     scale_strides: tuple[int, int] = (0, 0),
 ) -> LikSeqs:
-    s = LikSeqs()
-    s.data = data.data_ptr()
-    s.dtype = DTYPE_CODE[data.dtype]
-    s.dim = data.shape[-1]
-    s.n = n
-    s.len = length
-    s.stride_n = stride_n
-    s.stride_l = stride_l
-    s.cu_seqlens = ptr(cu)
-    s.lengths = ptr(lengths)
-    s.mask = ptr(mask)
-    s.mask_stride_n, s.mask_stride_l = mask_strides
-    s.token_scale = ptr(token_scale)
-    s.scale_stride_n, s.scale_stride_l = scale_strides
-    return s
+    return LikSeqs(
+        data.data_ptr(), DTYPE_CODE[data.dtype], data.shape[-1], n, length, stride_n, stride_l,
+        None if cu is None else cu.data_ptr(), None if lengths is None else lengths.data_ptr(),
+        None if mask is None else mask.data_ptr(), mask_strides[0], mask_strides[1],
+        None if token_scale is None else token_scale.data_ptr(), scale_strides[0], scale_strides[1],
+    )
 
 
 def version() -> str:
@@ -421,16 +433,11 @@ def call_opts():
     return ctypes.pointer(s)
 
 
-def _elem_align(dtype: torch.dtype) -> int:
-    """Elements per 16-byte chunk: the kernels need rows of whole chunks."""
-    return 16 // torch.empty((), dtype=dtype).element_size()
-
-
 def prepare_tokens(x: torch.Tensor) -> torch.Tensor:
     """Return ``x`` with a contiguous last dim padded (with zeros) to a multiple
     of 16 bytes, rows 16-byte aligned. Zero padding changes no dot product and
     no norm, so results are unaffected."""
-    align = _elem_align(x.dtype)
+    align = 16 // x.element_size()  # elements per 16-byte chunk: the kernels need rows of whole chunks
     d = x.shape[-1]
     pad = (-d) % align
     if pad:

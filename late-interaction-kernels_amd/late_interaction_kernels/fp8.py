@@ -42,7 +42,7 @@ def _quantize_kernel(X: torch.Tensor, dtype: torch.dtype, per_token: bool):
     lib = _lib.load()
     nbytes = lib.lik_quantize_fp8_workspace_size(flags)
     ws = _lib.workspace(nbytes, X.device)
-    with torch.cuda.device(X.device):
+    with _lib.on_device(X.device):
         rc = lib.lik_quantize_fp8(X.data_ptr(), _lib.DTYPE_CODE[X.dtype], X.numel() // d, d, flags, out.data_ptr(),
                                   scale.data_ptr(), _lib.ptr(ws), nbytes, _lib.stream_of(out))
     _lib.check(rc, "lik_quantize_fp8")

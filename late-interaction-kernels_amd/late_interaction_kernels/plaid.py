@@ -25,7 +25,7 @@ import ctypes
 import torch
 
 from . import _lib
-from ._core import assert_max_seqlen_covers
+from ._core import assert_max_seqlens_cover
 from .topk import topk_update
 
 _CENT_CODE = {torch.bfloat16: _lib.LIK_BF16, torch.float16: _lib.LIK_F16, torch.float32: _lib.LIK_F32}
@@ -58,7 +58,7 @@ def plaid_approx_score(
     if B == 0:
         return out
     lib = _lib.load()
-    with torch.cuda.device(codes.device):
+    with _lib.on_device(codes.device):
         rc = lib.lik_plaid_approx_score(
             qcs.data_ptr(), n_cent, Lq, qcs.stride(0), qcs.stride(1), codes.data_ptr(), B, L,
             codes.stride(0), lens.data_ptr(), out.data_ptr(), _lib.stream_of(out),
@@ -91,7 +91,7 @@ def _plaid_launch(Q, docs: _lib.LikPlaidDocs, normalize: bool, out: torch.Tensor
         Qc = Q[:, s0 : s0 + step]
         qs = _lib.seqs(Qc, n=Nq, length=Qc.shape[1], stride_n=Qc.stride(0), stride_l=Qc.stride(1))
         dst = out if n == 0 else tmp
-        with torch.cuda.device(Q.device):
+        with _lib.on_device(Q.device):
             rc = lib.lik_plaid_maxsim_ex(
                 ctypes.byref(qs), ctypes.byref(docs), flags, dst.data_ptr(), dst.stride(0), dst.stride(1),
                 _lib.call_opts(), _lib.stream_of(dst),
@@ -229,7 +229,7 @@ def maxsim_residual_varlen(
     cu = cu_seqlens_d.contiguous().to(torch.int32)
     Nd = cu.numel() - 1
     if max_seqlen_d is not None:
-        assert_max_seqlen_covers(cu, int(max_seqlen_d), "max_seqlen_d")
+        assert_max_seqlens_cover((cu, int(max_seqlen_d), "max_seqlen_d"))
     if torch.is_grad_enabled() and Q.requires_grad and Nq and Nd > 0 and Lq and codes_flat.numel():
         out = _residual_with_q_grad(Q, codes_flat, residuals_flat, centroids, bw, nbits, cu=cu, Nd=Nd, L=0,
                                     normalize=normalize)
@@ -342,7 +342,7 @@ class _ResidualQGradFn(torch.autograd.Function):
         lib = _lib.load()
         nbytes = lib.lik_maxsim_workspace_size(ctypes.byref(qs), ctypes.byref(ds), flags)
         ws = _lib.workspace(nbytes, Q.device)
-        with torch.cuda.device(Q.device):
+        with _lib.on_device(Q.device):
             rc = lib.lik_maxsim_argmax(ctypes.byref(qs), ctypes.byref(ds), flags, out.data_ptr(), out.stride(0),
                                        out.stride(1), argmax.data_ptr(), _lib.ptr(ws), nbytes, _lib.stream_of(out))
         _lib.check(rc, "lik_maxsim_argmax")
@@ -367,7 +367,7 @@ class _ResidualQGradFn(torch.autograd.Function):
         lib = _lib.load()
         nbytes = lib.lik_maxsim_backward_workspace_size(ctypes.byref(qs), ctypes.byref(ds), flags)
         ws = _lib.workspace(nbytes, Qp.device)
-        with torch.cuda.device(Qp.device):
+        with _lib.on_device(Qp.device):
             rc = lib.lik_maxsim_backward(g.data_ptr(), g.stride(0), ctypes.byref(qs), ctypes.byref(ds),
                                          argmax.data_ptr(), flags, gq.data_ptr(), None, _lib.ptr(ws), nbytes,
                                          _lib.stream_of(gq))
@@ -384,7 +384,7 @@ def _residual_with_q_grad(Q, codes_flat, residuals, centroids, bw, nbits, *, cu=
 
 def _decode_into(docs: _lib.LikPlaidDocs, t0: int, t1: int, normalize: bool, out: torch.Tensor) -> None:
     lib = _lib.load()
-    with torch.cuda.device(out.device):
+    with _lib.on_device(out.device):
         rc = lib.lik_plaid_decode(
             ctypes.byref(docs), t0, t1, _lib.LIK_NORMALIZE if normalize else 0, _lib.DTYPE_CODE[out.dtype],
             out.data_ptr(), out.stride(0), _lib.stream_of(out),
@@ -414,7 +414,7 @@ def _decoded_chunk_scores(Qp, docs, cu, j0: int, j1: int, t0: int, t1: int, norm
     opts = _lib.call_opts()
     nbytes = lib.lik_maxsim_workspace_size_ex(ctypes.byref(qs), ctypes.byref(ds), flags, opts)
     ws = _lib.workspace(nbytes, Qp.device)
-    with torch.cuda.device(Qp.device):
+    with _lib.on_device(Qp.device):
         rc = lib.lik_maxsim_ex(ctypes.byref(qs), ctypes.byref(ds), flags, 1.0, out.data_ptr(), out.stride(0),
                                out.stride(1), _lib.ptr(ws), nbytes, opts, _lib.stream_of(out))
     _lib.check(rc, "lik_maxsim")
@@ -532,7 +532,7 @@ class ResidualIndex:
         if T:
             docs = self._docs()
             lib = _lib.load()
-            with torch.cuda.device(self.codes.device):
+            with _lib.on_device(self.codes.device):
                 rc = lib.lik_plaid_token_records(ctypes.byref(docs), 0, T, self.token_rec.data_ptr(),
                                                  _lib.stream_of(self.token_rec))
             _lib.check(rc, "lik_plaid_token_records")
@@ -589,7 +589,7 @@ class ResidualIndex:
             nbytes = lib.lik_plaid_maxsim_qc_workspace_size(ctypes.byref(qs), ctypes.byref(docs))
             ws = _lib.workspace(nbytes, Q.device)
             flags = (_lib.LIK_NORMALIZE if normalize else 0) | _lib.LIK_TOKEN_RECORDS
-            with torch.cuda.device(Q.device):
+            with _lib.on_device(Q.device):
                 rc = lib.lik_plaid_maxsim_qc(ctypes.byref(qs), ctypes.byref(docs), self.token_rec.data_ptr(), flags,
                                              out.data_ptr(), out.stride(0), out.stride(1), _lib.ptr(ws), nbytes,
                                              _lib.call_opts(), _lib.stream_of(out))

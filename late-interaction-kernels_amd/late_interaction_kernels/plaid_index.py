@@ -48,7 +48,7 @@ def reverse_residual_bits(residuals: torch.Tensor) -> torch.Tensor:
     src = residuals.contiguous()
     out = torch.empty_like(src)
     lib = _lib.load()
-    with torch.cuda.device(src.device):
+    with _lib.on_device(src.device):
         rc = lib.lik_residual_reverse_bits(src.data_ptr(), out.data_ptr(), src.numel(), _lib.stream_of(out))
     _lib.check(rc, "lik_residual_reverse_bits")
     return out

@@ -7,7 +7,7 @@ from __future__ import annotations
 
 import torch
 
-from ._core import (assert_max_seqlen_covers, pairs_backward, pairs_maxsim, pairs_maxsim_train, seqlen_max,
+from ._core import (assert_max_seqlens_cover, pairs_backward, pairs_maxsim, pairs_maxsim_train, seqlen_max,
                     unify_dtype)
 from .autograd import _needs_grad
 
@@ -65,11 +65,11 @@ def score_pairs_packed(
     cu_q = cu_seqlens_q.to(torch.int32).contiguous()
     cu_d = cu_seqlens_d.to(torch.int32).contiguous()
     if max_seqlen_q is None:
+        assert_max_seqlens_cover((cu_d, None if max_seqlen_d is None else int(max_seqlen_d), "max_seqlen_d"))
         max_seqlen_q = seqlen_max(cu_q)
     else:
-        assert_max_seqlen_covers(cu_q, int(max_seqlen_q), "max_seqlen_q")
-    if max_seqlen_d is not None:
-        assert_max_seqlen_covers(cu_d, int(max_seqlen_d), "max_seqlen_d")
+        assert_max_seqlens_cover((cu_q, int(max_seqlen_q), "max_seqlen_q"),
+                                 (cu_d, None if max_seqlen_d is None else int(max_seqlen_d), "max_seqlen_d"))
     Qp, Dp = unify_dtype(Q_packed, D_packed)
     if _needs_grad(Q_packed, D_packed):
         if Qp.dtype == torch.float64:

@@ -57,7 +57,7 @@ def topk_update(
         return out_s, out_i
     nws = lib.lik_topk_select_workspace_size(R, n, kk)
     ws = torch.empty(nws, device=dev, dtype=torch.uint8) if nws else None
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = lib.lik_topk_select(
             cs.data_ptr(), R, n, cs.stride(0), idx_base,
             _lib.ptr(run_s), _lib.ptr(run_i), pk, run_s.stride(0) if run_s is not None else 0,
