@@ -8,9 +8,14 @@
 // "better score, then lower index", so the k best candidates are exactly the
 // k largest keys and any grouping of the candidates selects the same set.
 //
-// One workgroup selects the kk largest of up to MAX_KEYS LDS-resident keys
-// by an 8-pass MSB-first radix select (256-bin histograms), compacts the
-// winners and bitonic-sorts them. A row wider than one workgroup's share is
+// One workgroup selects the kk largest of up to MAX_KEYS LDS-resident keys by
+// histogram passes of 2048 bins over the keys' own range (then over the bin that
+// holds the kk-th largest), compacts the winners and puts each at its rank (up
+// to 256 of them; more are bitonic-sorted). Latency is what bounds it: a
+// barrier per step and few keys per thread. (Byte-wise passes from the top, whose
+// first ones put all scores of a call in one bin, and a bitonic sort took 17.3 us
+// for 16 rows of 4096 scores at k = 100, 25 + 20 us for the two levels of 100,000
+// scores; now 13.8, and 19 + 12.) A row wider than one workgroup's share is
 // reduced as a tree: level 0 gives each MAX_N-score slice of a row its own
 // workgroup, which writes its k best keys (0-padded) to a workspace; each
 // further level merges up to MAX_KEYS / k such lists per workgroup, and the
@@ -23,6 +28,7 @@
 namespace lik {
 
 constexpr int TK_THREADS = 256;
+constexpr int TK_BIN_BITS = 11, TK_BINS = 1 << TK_BIN_BITS;  // of one selection pass
 // Two LDS capacity classes. Small (k <= 1024): 4096 scores per level-0 group
 // plus a running list, winners sorted in their own array (48 KB). Large
 // (k <= 8192): 16384 keys (128 KB, one workgroup per CU), 8192 scores per
@@ -82,11 +88,11 @@ __global__ void __launch_bounds__(TK_THREADS) topk_select_kernel(TopkArgs a) {
   __shared__ uint64_t s_keys[C::MAX_KEYS];
   __shared__ uint64_t s_sel_own[C::INPLACE ? 1 : C::MAX_K];
   uint64_t* const s_sel = C::INPLACE ? s_keys : s_sel_own;
-  __shared__ uint32_t s_hist[256];
-  __shared__ uint64_t s_prefix, s_pmask;
+  __shared__ uint32_t s_hist[TK_BINS];
+  __shared__ uint64_t s_lo;
   __shared__ int s_kk, s_done, s_cnt, s_real, s_fcnt;
   __shared__ int s_wcnt[TK_THREADS / 64];
-  __shared__ uint64_t s_wmin[TK_THREADS / 64];
+  __shared__ uint64_t s_wmin[TK_THREADS / 64], s_wmax[TK_THREADS / 64];
 
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int64_t row = blockIdx.x / a.groups;
@@ -161,71 +167,97 @@ __global__ void __launch_bounds__(TK_THREADS) topk_select_kernel(TopkArgs a) {
       if (lane == 0 && nz) atomicAdd(&s_real, __popcll(nz));
     }
   }
-  if (tid == 0) {
-    s_prefix = 0;
-    s_pmask = 0;
-    s_done = 0;
-    s_cnt = 0;
-  }
+  if (tid == 0) s_cnt = 0;
   __syncthreads();
   const int kk_sel = (int)min(a.k, (int64_t)s_real);
-  if (tid == 0) s_kk = kk_sel;
-  __syncthreads();
 
   if (kk_sel > 0) {
-    for (int pass = 0; pass < 8; ++pass) {
-      const int shift = 56 - 8 * pass;
-      s_hist[tid] = 0;  // TK_THREADS == 256 bins
+    // smallest and largest real key
+    uint64_t mn = ~0ull, mx = 0;
+    for (int i = tid; i < total; i += TK_THREADS) {
+      const uint64_t key = s_keys[i];
+      if (key != 0) {
+        mn = key < mn ? key : mn;
+        mx = key > mx ? key : mx;
+      }
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+      const uint64_t x = __shfl_xor(mn, o), y = __shfl_xor(mx, o);
+      mn = x < mn ? x : mn;
+      mx = y > mx ? y : mx;
+    }
+    if (lane == 0) {
+      s_wmin[wv] = mn;
+      s_wmax[wv] = mx;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < TK_THREADS / 64; ++w) {
+      mn = s_wmin[w] < mn ? s_wmin[w] : mn;
+      mx = s_wmax[w] > mx ? s_wmax[w] : mx;
+    }
+    // Passes over the keys in [lo, lo + nbins << shift): lo and shift follow
+    // the keys' own range, so the first pass already spreads them over the
+    // bins (scores of one call share their leading bits).
+    uint64_t lo = mn, nbins = TK_BINS;
+    const uint64_t span = mx - mn;
+    int shift = span ? 64 - __builtin_clzll(span) - TK_BIN_BITS : 0;
+    shift = shift < 0 ? 0 : shift;
+    uint32_t kk = (uint32_t)kk_sel;
+    for (;;) {
+      for (int i = tid; i < TK_BINS; i += TK_THREADS) s_hist[i] = 0;
       __syncthreads();
-      const uint64_t prefix = s_prefix, pmask = s_pmask;
       for (int i = tid; i < total; i += TK_THREADS) {
         const uint64_t key = s_keys[i];
-        if ((key & pmask) == prefix) atomicAdd(&s_hist[(key >> shift) & 255u], 1u);
+        const uint64_t bin = (key - lo) >> shift;
+        if (key >= lo && bin < nbins) atomicAdd(&s_hist[bin], 1u);
       }
       __syncthreads();
-      if (wv == 0) {
-        // lane l owns bins 255-4l .. 252-4l (descending); find the bin holding
-        // the kk-th largest remaining key with a wavefront inclusive scan.
-        uint32_t c[4], local = 0;
+      // thread t owns 8 bins from TK_BINS - 1 - 8 t down; one of them finds the
+      // bin holding the kk-th largest key of the range
+      constexpr int BPT = TK_BINS / TK_THREADS;
+      uint32_t c[BPT], local = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          c[j] = s_hist[255 - 4 * lane - j];
-          local += c[j];
-        }
-        uint32_t incl = local;
+      for (int j = 0; j < BPT; ++j) {
+        c[j] = s_hist[TK_BINS - 1 - BPT * tid - j];
+        local += c[j];
+      }
+      uint32_t incl = local;
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-          const uint32_t v = __shfl_up(incl, o);
-          if (lane >= o) incl += v;
-        }
-        const uint32_t excl = incl - local;
-        const uint32_t kk = (uint32_t)s_kk;
-        if (excl < kk && kk <= incl) {
-          uint32_t cum = excl;
-          int bin = 0;
-          uint32_t rem = 0, cnt = 0;
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t v = __shfl_up(incl, o);
+        if (lane >= o) incl += v;
+      }
+      if (lane == 63) s_wcnt[wv] = (int)incl;
+      __syncthreads();
+      for (int w = 0; w < wv; ++w) incl += (uint32_t)s_wcnt[w];
+      const uint32_t excl = incl - local;
+      if (excl < kk && kk <= incl) {
+        uint32_t cum = excl;
+        bool found = false;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            if (cnt == 0 && cum + c[j] >= kk) {
-              bin = 255 - 4 * lane - j;
-              rem = kk - cum;
-              cnt = c[j];
-            }
-            cum += c[j];
+        for (int j = 0; j < BPT; ++j) {
+          if (!found && cum + c[j] >= kk) {
+            found = true;
+            s_lo = lo + ((uint64_t)(TK_BINS - 1 - BPT * tid - j) << shift);
+            s_kk = (int)(kk - cum);
+            s_done = c[j] == kk - cum ? 1 : 0;
           }
-          s_prefix = prefix | ((uint64_t)bin << shift);
-          s_pmask = pmask | ((uint64_t)0xffu << shift);
-          s_kk = (int)rem;
-          s_done = (cnt == rem) ? 1 : 0;
+          cum += c[j];
         }
       }
       __syncthreads();
-      if (s_done) break;
+      lo = s_lo;
+      kk = (uint32_t)s_kk;
+      if (s_done || shift == 0) break;  // (at shift 0 a bin holds one key: keys are unique)
+      const int next = shift > TK_BIN_BITS ? shift - TK_BIN_BITS : 0;
+      nbins = 1ull << (shift - next);
+      shift = next;
     }
 
-    // winners: (key & pmask) >= prefix; exactly kk_sel of them (keys are
-    // unique and the kk_sel-th largest is a real key, above every 0 pad)
-    const uint64_t prefix = s_prefix, pmask = s_pmask;
+    // winners: key >= lo; exactly kk_sel of them (keys are unique and the
+    // kk_sel-th largest is a real key, above every 0 pad)
     if constexpr (C::INPLACE) {
       // In place, one 256-key chunk at a time: every key of the chunk is read
       // before any write, and a winner's slot is below the number of keys
@@ -234,7 +266,7 @@ __global__ void __launch_bounds__(TK_THREADS) topk_select_kernel(TopkArgs a) {
       for (int i0 = 0; i0 < total; i0 += TK_THREADS) {
         const int i = i0 + tid;
         const uint64_t key = i < total ? s_keys[i] : 0;
-        const bool win = i < total && (key & pmask) >= prefix;
+        const bool win = i < total && key >= lo;
         const uint64_t bal = __ballot(win);
         if (lane == 0) s_wcnt[wv] = (int)__popcll(bal);
         __syncthreads();
@@ -251,7 +283,7 @@ __global__ void __launch_bounds__(TK_THREADS) topk_select_kernel(TopkArgs a) {
     } else {
       for (int i = tid; i < total; i += TK_THREADS) {
         const uint64_t key = s_keys[i];
-        if ((key & pmask) >= prefix) {
+        if (key >= lo) {
           const int pos = atomicAdd(&s_cnt, 1);
           if (pos < C::MAX_K) s_sel[pos] = key;
         }
@@ -259,6 +291,29 @@ __global__ void __launch_bounds__(TK_THREADS) topk_select_kernel(TopkArgs a) {
     }
   }
   __syncthreads();
+  auto put = [&](int64_t at, uint64_t key) {
+    if (a.keys_out) {
+      a.keys_out[((int64_t)blockIdx.x) * a.k + at] = key;
+      return;
+    }
+    uint32_t o = (uint32_t)(key >> 32);
+    if (!a.largest) o = ~o;
+    a.out_s[row * a.old + at] = order_float(o);
+    a.out_i[row * a.old + at] = (int64_t)(uint32_t)(~(uint32_t)key);
+  };
+  if (a.keys_out)
+    for (int i = kk_sel + tid; i < a.k; i += TK_THREADS) put(i, 0);
+  if (kk_sel <= TK_THREADS) {
+    // a winner's place is the number of larger ones (the reads are broadcasts)
+    if (tid < kk_sel) {
+      const uint64_t key = s_sel[tid];
+      int rank = 0;
+#pragma unroll 8
+      for (int i = 0; i < kk_sel; ++i) rank += s_sel[i] > key ? 1 : 0;
+      put(rank, key);
+    }
+    return;
+  }
   int P = 1;
   while (P < kk_sel) P <<= 1;
   for (int i = kk_sel + tid; i < P; i += TK_THREADS) s_sel[i] = 0;
@@ -279,18 +334,7 @@ __global__ void __launch_bounds__(TK_THREADS) topk_select_kernel(TopkArgs a) {
       __syncthreads();
     }
   }
-  if (a.keys_out) {
-    uint64_t* dst = a.keys_out + ((int64_t)blockIdx.x) * a.k;
-    for (int i = tid; i < a.k; i += TK_THREADS) dst[i] = i < kk_sel ? s_sel[i] : 0;
-  } else {
-    for (int i = tid; i < kk_sel; i += TK_THREADS) {
-      const uint64_t key = s_sel[i];
-      uint32_t o = (uint32_t)(key >> 32);
-      if (!a.largest) o = ~o;
-      a.out_s[row * a.old + i] = order_float(o);
-      a.out_i[row * a.old + i] = (int64_t)(uint32_t)(~(uint32_t)key);
-    }
-  }
+  for (int i = tid; i < kk_sel; i += TK_THREADS) put(i, s_sel[i]);
 }
 
 // Tree shape for one call: level-0 groups, lists merged per later group, and
