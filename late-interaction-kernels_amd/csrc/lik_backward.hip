@@ -1196,6 +1196,91 @@ __global__ void __launch_bounds__(256) bucket_ptr_kernel(const int32_t* sorted, 
   ptr[k] = (int32_t)lo;
 }
 
+// Both pair lists in one launch for up to kListPairs pairs over at most kListKeys
+// owners: workgroup 0 the queries', 1 the docs'. A stable counting sort in LDS:
+// each wavefront counts, then places, its own contiguous share of the pairs, so
+// an owner's pairs keep increasing pair order. (The device radix sorts and
+// their key and pointer kernels are nine launches, 36 us for 4096 pairs and as
+// much again in gaps; this one takes 11.)
+constexpr int kListPairs = 16384, kListKeys = 2048;
+__global__ void __launch_bounds__(1024) pair_lists_kernel(const int32_t* pair_q, const int32_t* pair_d, int np, int nq,
+                                                          int nd, int32_t* q_ptr, int32_t* q_list, int32_t* d_ptr,
+                                                          int32_t* d_list) {
+  constexpr int NW = 16, NT = 1024, CH = kListPairs / NT, RPT = kListKeys / NT;
+  __shared__ __attribute__((aligned(16))) uint16_t s_cnt[NW][kListKeys];
+  __shared__ int s_tot[NW];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const bool docs = blockIdx.x != 0;
+  const int n = docs ? nd : nq;
+  int32_t* const ptr = docs ? d_ptr : q_ptr;
+  int32_t* const list = docs ? d_list : q_list;
+  for (int k = tid; k < NW * kListKeys / 2; k += NT) ((uint32_t*)s_cnt)[k] = 0u;
+  const int share = (np + NT - 1) / NT * 64;  // pairs per wavefront
+  int key[CH];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int p = wv * share + c * 64 + lane;
+    key[c] = -1;
+    if (c * 64 < share && p < np) {
+      const int q = pair_q[p], d = pair_d[p];
+      if (q >= 0 && q < nq && d >= 0 && d < nd) key[c] = docs ? d : q;  // out of range: in no list
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+    if (key[c] >= 0) atomicAdd((uint32_t*)s_cnt[wv] + (key[c] >> 1), 1u << (16 * (key[c] & 1)));
+  __syncthreads();
+  int mine = 0;
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) {
+    const int k = tid * RPT + r;
+    if (k < n)
+      for (int w = 0; w < NW; ++w) mine += s_cnt[w][k];
+  }
+  int incl = mine;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int t = __shfl_up(incl, o);
+    if (lane >= o) incl += t;
+  }
+  if (lane == 63) s_tot[wv] = incl;
+  __syncthreads();
+  int base = incl - mine;
+  for (int w = 0; w < wv; ++w) base += s_tot[w];
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) {
+    const int k = tid * RPT + r;
+    if (k < n) {
+      ptr[k] = base;
+      for (int w = 0; w < NW; ++w) {
+        const int m = s_cnt[w][k];
+        s_cnt[w][k] = (uint16_t)base;
+        base += m;
+      }
+      if (k == n - 1) ptr[n] = base;
+    }
+  }
+  __syncthreads();
+  const int kbits = 32 - __builtin_clz(n);  // keys are below n
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    if (c * 64 >= share) break;
+    uint64_t same = __ballot(key[c] >= 0);  // lanes with this lane's key
+    for (int b = 0; b < kbits; ++b) {
+      const bool on = (key[c] >> b) & 1;
+      const uint64_t m = __ballot(on);
+      same &= on ? m : ~m;
+    }
+    if (key[c] >= 0) {
+      const int rank = (int)__popcll(same & ((1ull << lane) - 1ull));
+      const int pos = s_cnt[wv][key[c]] + rank;
+      list[pos] = wv * share + c * 64 + lane;
+      if (rank == 0) s_cnt[wv][key[c]] = (uint16_t)(pos + (int)__popcll(same));
+    }
+  }
+}
+
 struct PairWs {
   size_t kq, kd, iota, ks, qlist, dlist, qptr, dptr, temp, temp_bytes, total;
 };
@@ -1476,22 +1561,28 @@ int lik_maxsim_pairs_backward(const float* grad, const lik_seqs_t* Q, const lik_
   if ((size_t)(ws - (char*)workspace) + w.total - 256 > workspace_bytes) return LIK_ERR_WORKSPACE;
   hipStream_t s = (hipStream_t)stream;
   auto I = [&](size_t off) { return (int32_t*)(ws + off); };
-  const unsigned pb = (unsigned)((num_pairs + 255) / 256);
-  hipLaunchKernelGGL(pair_keys_kernel, dim3(pb), dim3(256), 0, s, pair_q, pair_d, num_pairs, Q->n, D->n, I(w.kq),
-                     I(w.kd), I(w.iota));
-  if (hipGetLastError() != hipSuccess) return LIK_ERR_LAUNCH;
-  const int eb_bits = end_bit_for(Q->n > D->n ? Q->n : D->n);
-  // stable LSD radix sort: pairs of one owner keep increasing pair order
-  struct Pass { size_t key, list, ptr; int64_t n; } passes[2] = {{w.kq, w.qlist, w.qptr, Q->n},
-                                                               {w.kd, w.dlist, w.dptr, D->n}};
-  for (const Pass& ps : passes) {
-    size_t tb = w.temp_bytes;
-    if (hipcub::DeviceRadixSort::SortPairs(ws + w.temp, tb, I(ps.key), I(w.ks), I(w.iota), I(ps.list),
-                                           (int)num_pairs, 0, eb_bits, s) != hipSuccess)
-      return LIK_ERR_LAUNCH;
-    hipLaunchKernelGGL(bucket_ptr_kernel, dim3((unsigned)((ps.n + 1 + 255) / 256)), dim3(256), 0, s, I(w.ks),
-                       num_pairs, ps.n, I(ps.ptr));
+  if (num_pairs <= kListPairs && Q->n <= kListKeys && D->n <= kListKeys) {
+    hipLaunchKernelGGL(pair_lists_kernel, dim3(2), dim3(1024), 0, s, pair_q, pair_d, (int)num_pairs, (int)Q->n,
+                       (int)D->n, I(w.qptr), I(w.qlist), I(w.dptr), I(w.dlist));
     if (hipGetLastError() != hipSuccess) return LIK_ERR_LAUNCH;
+  } else {
+    const unsigned pb = (unsigned)((num_pairs + 255) / 256);
+    hipLaunchKernelGGL(pair_keys_kernel, dim3(pb), dim3(256), 0, s, pair_q, pair_d, num_pairs, Q->n, D->n, I(w.kq),
+                       I(w.kd), I(w.iota));
+    if (hipGetLastError() != hipSuccess) return LIK_ERR_LAUNCH;
+    const int eb_bits = end_bit_for(Q->n > D->n ? Q->n : D->n);
+    // stable LSD radix sort: pairs of one owner keep increasing pair order
+    struct Pass { size_t key, list, ptr; int64_t n; } passes[2] = {{w.kq, w.qlist, w.qptr, Q->n},
+                                                                 {w.kd, w.dlist, w.dptr, D->n}};
+    for (const Pass& ps : passes) {
+      size_t tb = w.temp_bytes;
+      if (hipcub::DeviceRadixSort::SortPairs(ws + w.temp, tb, I(ps.key), I(w.ks), I(w.iota), I(ps.list),
+                                             (int)num_pairs, 0, eb_bits, s) != hipSuccess)
+        return LIK_ERR_LAUNCH;
+      hipLaunchKernelGGL(bucket_ptr_kernel, dim3((unsigned)((ps.n + 1 + 255) / 256)), dim3(256), 0, s, I(w.ks),
+                         num_pairs, ps.n, I(ps.ptr));
+      if (hipGetLastError() != hipSuccess) return LIK_ERR_LAUNCH;
+    }
   }
   BwdParams bp{};
   bp.qsplit = 1;
