@@ -73,16 +73,16 @@ __global__ void __launch_bounds__(256) doc_extent_kernel(const int8_t* mask, int
   }
 }
 
-// The same summary for masks whose token bytes are contiguous (stride 1),
-// with 4-byte-aligned rows, L <= 1024 and the whole mask under 4 GB. The
-// byte-per-lane form spends ~90 instructions of a 64-lane wavefront per doc
-// (and one load round trip per doc); here 16 lanes take a doc, 4 docs per
-// wavefront, and lane q reads tokens 16 q .. 16 q + 15 of each 256-token pass
-// as four dwords, all of a wavefront's loads issued before any is used. The
-// nonzero bytes of a dword become 4 bits by an or-fold and one multiply. The
-// loads go through a buffer resource that ends at the mask's last byte (a
-// dword past it reads as 0; bytes past a doc's length are dropped by the
-// length test).
+// The same summary for masks whose token bytes are contiguous (stride 1), L <=
+// 256 NP and the whole mask under 2 GB. The byte-per-lane form spends ~90
+// instructions of a 64-lane wavefront per doc (and one load round trip per
+// doc); here 16 lanes take a doc, 4 docs per wavefront, and lane q reads tokens
+// 16 q .. 16 q + 15 of each 256-token pass as four dwords, all of a wavefront's
+// loads issued before any is used. Rows that do not start on 4 bytes (UNAL: an
+// odd row length, a page image's 1030) read the five dwords that cover them and
+// shift. The nonzero bytes of a dword become 4 bits by an or-fold and one
+// multiply. The loads go through a buffer resource over the aligned dwords that
+// hold the mask (bytes past a doc's length are dropped by the length test).
 __device__ __forceinline__ uint32_t nonzero_bytes4(uint32_t x) {
   uint32_t y = x | (x >> 4);
   y |= y >> 2;
@@ -92,11 +92,12 @@ __device__ __forceinline__ uint32_t nonzero_bytes4(uint32_t x) {
   return ((y * 0x01020408u) >> 24) & 0xfu;
 }
 
-__global__ void __launch_bounds__(256) doc_extent_w4_kernel(const int8_t* mask, int64_t msn, uint32_t mbytes,
-                                                            int64_t n, int L, const int32_t* lengths,
+template <int NP, bool UNAL>  // 256-token passes
+__global__ void __launch_bounds__(256) doc_extent_w4_kernel(const int8_t* mask, int64_t msn, uint32_t skew,
+                                                            uint32_t mbytes, int64_t n, int L, const int32_t* lengths,
                                                             int32_t* extent, uint8_t* holes, uint32_t* tbits,
                                                             int tbits_sn) {
-  constexpr int NP = 4;  // 256-token passes (L <= 1024)
+  // mask: the 4-byte boundary `skew` bytes before the mask's first byte
   const int lane = threadIdx.x & 63, q = lane & 15;
   const int64_t j = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 4 + (lane >> 4);
   const int np = (L + 255) >> 8;  // passes that hold tokens (uniform)
@@ -107,15 +108,24 @@ __global__ void __launch_bounds__(256) doc_extent_w4_kernel(const int8_t* mask, 
   }
   const __amdgpu_buffer_rsrc_t rs =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(mask), (short)0, (int)mbytes, 0x00020000);
-  const uint32_t row = j < n ? (uint32_t)(j * msn) : 0u;
-  uint32_t w[NP][4];
+  const uint32_t row = j < n ? skew + (uint32_t)(j * msn) : 0u;
+  const uint32_t row4 = row & ~3u, shift = row & 3u;
+  constexpr int ND = UNAL ? 5 : 4;
+  uint32_t w[NP][ND];
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int t = p * 256 + q * 16 + 4 * i;
-      w[p][i] = (p < np && t < Lj) ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, row + (uint32_t)t, 0, 0) : 0u;
+    for (int i = 0; i < ND; ++i) {
+      const int t = p * 256 + q * 16 + 4 * i;  // dword i holds tokens t - shift .. t - shift + 3
+      w[p][i] = (p < np && t < Lj + (UNAL ? 3 : 0))
+                    ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, row4 + (uint32_t)t, 0, 0) : 0u;
     }
+  }
+  if constexpr (UNAL) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w[p][i] = __builtin_amdgcn_alignbyte(w[p][i + 1], w[p][i], shift);
   }
   int last = -1, cnt = 0;
 #pragma unroll
@@ -646,12 +656,18 @@ int maxsim_impl(const lik_seqs_t* Q, const lik_seqs_t* D, uint32_t flags, float 
     p.tbits = (const uint32_t*)(ws + wl.tbits_off);
     p.tbits_sn = (D->len + 31) / 32;
     const int64_t mend = (D->n - 1) * D->mask_stride_n + D->len;  // one past the mask's last byte
-    if (D->mask_stride_l == 1 && D->mask_stride_n >= 0 && D->mask_stride_n % 4 == 0 &&
-        (uintptr_t)D->mask % 4 == 0 && D->len <= 1024 && mend < 0x7fffffffLL)
-      hipLaunchKernelGGL(doc_extent_w4_kernel, dim3((unsigned)((D->n + 15) / 16)), dim3(256), 0, s, D->mask,
-                         D->mask_stride_n, (uint32_t)mend, D->n, (int)D->len, D->lengths,
+    const uint32_t skew = (uint32_t)((uintptr_t)D->mask & 3);
+    const bool w4 = D->mask_stride_l == 1 && D->mask_stride_n >= 0 && D->len <= 2048 && mend + 8 < 0x7fffffffLL;
+    auto launch_w4 = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)((D->n + 15) / 16)), dim3(256), 0, s, D->mask - skew, D->mask_stride_n,
+                         skew, (uint32_t)(skew + mend + 3) & ~3u, D->n, (int)D->len, D->lengths,
                          (int32_t*)(ws + wl.extent_off), (uint8_t*)(ws + wl.holes_off),
                          (uint32_t*)(ws + wl.tbits_off), (int)p.tbits_sn);
+    };
+    const bool al4 = skew == 0 && D->mask_stride_n % 4 == 0;
+    // (1024 docs of 1030 tokens: 10.3 us on the byte-per-lane kernel, 7.0 here)
+    if (w4 && D->len <= 1024) al4 ? launch_w4(doc_extent_w4_kernel<4, false>) : launch_w4(doc_extent_w4_kernel<4, true>);
+    else if (w4) al4 ? launch_w4(doc_extent_w4_kernel<8, false>) : launch_w4(doc_extent_w4_kernel<8, true>);
     else
       hipLaunchKernelGGL(doc_extent_kernel, dim3((unsigned)((D->n + 3) / 4)), dim3(256), 0, s, D->mask,
                          D->mask_stride_n, D->mask_stride_l, D->n, D->len, D->lengths,
