@@ -412,18 +412,19 @@ int pick_R(int64_t ngroups, int64_t ndocs, int dpad, const lik_launch_opts_t* op
   } else if (ngroups > 1 && wg_cu > 0 && dpad > 0 && dpad <= 128) {
     // Several query blocks: a workgroup costs ~11 us of query-block load and
     // pipeline fill, as much as 250 doc tokens, so the docs are dealt out in
-    // whole rounds of the chip, one if that leaves at most 48 docs per
-    // workgroup, else rounds of about 32 docs (16 where the lengths vary as
-    // widely as packed corpora's do, so that the last round evens out). k
+    // whole rounds of the chip of up to 128 docs per workgroup (512 x 4096
+    // docs: 16 docs 2176 us, 32: 2150, 64: 2135, 128: 2126). Packed corpora, whose
+    // lengths vary more, take rounds of about 16 docs above 48, so that the
+    // last round evens out (8192 docs of 16 to 2048 tokens: 1390 us, 64: 1417). k
     // ranges per XCD: the k * ngroups workgroups there fill its 32 CUs.
     // Against ~2048 workgroups whatever the size: 256 x 32 query tokens, 256
     // docs of 50 to 300 tokens 131 -> 93 us (training forward 239 -> 153), 64
     // queries x 1000 docs 172 -> 96, fp8 64 x 24 tokens x 1000 pages 265 -> 223,
-    // fp32 32 queries x 2048 docs 464 -> 315; 512 x 4096 docs unchanged.
+    // fp32 32 queries x 2048 docs 464 -> 315.
     const int64_t slots = 32 * wg_cu;
     const int64_t k = slots > ngroups ? slots / ngroups : 1;
-    const int64_t per = (ndocs + 8 * k - 1) / (8 * k), len = packed ? 16 : 32;
-    const int64_t rounds = per > 48 ? (per + len - 1) / len : 1;
+    const int64_t per = (ndocs + 8 * k - 1) / (8 * k);
+    const int64_t rounds = packed ? (per > 48 ? (per + 15) / 16 : 1) : (per + 127) / 128;
     R = (ndocs + 8 * k * rounds - 1) / (8 * k * rounds);
   }
   if (opts && opts->docs_per_wg > 0) R = opts->docs_per_wg;  // caller-forced (lik_launch_opts_t)
