@@ -395,9 +395,10 @@ int make_plan(int dt, int dim, int64_t nq, int64_t lq, bool one_query_per_group,
 
 // Docs per workgroup. dpad > 0: a dense MaxSim launch of that row width (PLAID
 // tiles pass 0: their workgroups are latency-bound, more of them help).
-// wg_cu > 0: a cross product whose workgroups share a CU wg_cu at a time.
+// wg_cu > 0: a cross product of padded docs of len tokens whose workgroups share
+// a CU wg_cu at a time.
 int pick_R(int64_t ngroups, int64_t ndocs, int dpad, const lik_launch_opts_t* opts = nullptr, int wg_cu = 0,
-           bool packed = false) {
+           int64_t len = 0) {
   const int64_t target = 2048;
   int64_t R = (ndocs * ngroups) / target;
   if (ngroups == 1 && dpad > 0) {
@@ -411,21 +412,32 @@ int pick_R(int64_t ngroups, int64_t ndocs, int dpad, const lik_launch_opts_t* op
     if (r1 > R) R = r1;
   } else if (ngroups > 1 && wg_cu > 0 && dpad > 0 && dpad <= 128) {
     // Several query blocks: a workgroup costs ~11 us of query-block load and
-    // pipeline fill, as much as 250 doc tokens, so the docs are dealt out in
-    // whole rounds of the chip of up to 128 docs per workgroup (512 x 4096
-    // docs: 16 docs 2176 us, 32: 2150, 64: 2135, 128: 2126). Packed corpora, whose
-    // lengths vary more, take rounds of about 16 docs above 48, so that the
-    // last round evens out (8192 docs of 16 to 2048 tokens: 1390 us, 64: 1417). k
-    // ranges per XCD: the k * ngroups workgroups there fill its 32 CUs.
-    // Against ~2048 workgroups whatever the size: 256 x 32 query tokens, 256
-    // docs of 50 to 300 tokens 131 -> 93 us (training forward 239 -> 153), 64
-    // queries x 1000 docs 172 -> 96, fp8 64 x 24 tokens x 1000 pages 265 -> 223,
-    // fp32 32 queries x 2048 docs 464 -> 315.
+    // pipeline fill, as much as 8 tiles, so the docs are dealt out in whole
+    // rounds of the chip: with k doc ranges per XCD, k * ngroups workgroups
+    // share its 32 * wg_cu slots. Of 1 .. 16 rounds (k as large as they allow)
+    // the cheapest, counting the rounds' tiles and fills and, for the uneven end
+    // of the last one, a tenth of a workgroup's tiles. (Packed corpora keep ~2048
+    // workgroups: lengths that vary a hundredfold need more, shorter workgroups,
+    // by how much only the lengths tell: 33 queries x 500 docs of 16 to 2048
+    // tokens 128 us, this rule's 168 workgroups 171.) Against ~2048 workgroups
+    // whatever the size: 256 x 32 query tokens, 256 docs of 50 to 300 tokens 131 -> 93 us
+    // (training forward 239 -> 153), 64 queries x 1000 docs 172 -> 96, fp8 64 x 24
+    // tokens x 1000 pages 265 -> 223, fp32 32 queries x 2048 docs 464 -> 315; 512 x
+    // 4096 docs at 16 docs per workgroup 2176 us, 32: 2150, 64: 2135, 128: 2126.
     const int64_t slots = 32 * wg_cu;
-    const int64_t k = slots > ngroups ? slots / ngroups : 1;
-    const int64_t per = (ndocs + 8 * k - 1) / (8 * k);
-    const int64_t rounds = packed ? (per > 48 ? (per + 15) / 16 : 1) : (per + 127) / 128;
-    R = (ndocs + 8 * k * rounds - 1) / (8 * k * rounds);
+    const double tiles = (double)((len + 31) / 32) * 0.75;  // per doc, part of them masked
+    double best = 0.0;
+    const int64_t r0 = (ngroups + slots - 1) / slots;
+    for (int64_t r = r0; r < r0 + 16; ++r) {
+      const int64_t k = r * slots / ngroups;
+      const int64_t docs = (ndocs + 8 * k - 1) / (8 * k);
+      const double cost = r * (docs * tiles + 8.0) + 0.1 * docs * tiles;
+      if (r == r0 || cost < best) {
+        best = cost;
+        R = docs;
+      }
+      if (docs <= 1) break;
+    }
   }
   if (opts && opts->docs_per_wg > 0) R = opts->docs_per_wg;  // caller-forced (lik_launch_opts_t)
   if (R < 1) R = 1;
@@ -703,7 +715,7 @@ int maxsim_impl(const lik_seqs_t* Q, const lik_seqs_t* D, uint32_t flags, float 
     if (ps.d.lengths) ps.d.lengths += j0;
     if (ps.amax) ps.amax += j0 * ps.amax_ld;
     const bool two_wg = pl.W == 4 && pl.NSUB >= 4 && !argmax && !(ps.normalize & 2);
-    ps.R = pick_R(ps.ngroups, n, pl.dpad, opts, kd ? 0 : (two_wg ? 2 : 1), D->cu_seqlens != nullptr);
+    ps.R = pick_R(ps.ngroups, n, pl.dpad, opts, (kd || D->cu_seqlens) ? 0 : (two_wg ? 2 : 1), D->len);
     ps.NR = (n + ps.R - 1) / ps.R;
     ps.xcd_map = ps.NR >= 8 ? 1 : 0;
     const int64_t nb = ps.xcd_map ? ps.ngroups * ((ps.NR + 7) / 8) * 8 : ps.ngroups * ps.NR;
