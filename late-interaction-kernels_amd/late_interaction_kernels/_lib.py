@@ -263,19 +263,30 @@ def require_gpu(*tensors: torch.Tensor | None) -> None:
 def plain_op(*tensors: torch.Tensor) -> bool:
     """Whether a kernel may stand in for a chain of torch operators on these
     tensors: GPU tensors of torch's own class, no gradient or forward-mode
-    tangent to carry, nothing tracing, batching or intercepting the operators."""
+    tangent to carry, nothing tracing, batching or intercepting the operators.
+    (Torch has no public names for these states; a torch that lacks one of the
+    private ones asked here gets the operators.)"""
     if any(type(t) not in (torch.Tensor, torch.nn.Parameter) or t.device.type != "cuda" for t in tensors):
         return False
     if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
         return False
-    if torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.maybe_current_level() is not None:
+    try:
+        return not (torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.maybe_current_level() is not None
+                    or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                    or torch.jit.is_tracing() or torch.compiler.is_compiling())
+    except AttributeError:
         return False
-    return not (torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-                or torch.jit.is_tracing() or torch.compiler.is_compiling())
+
+
+# the current stream's handle and the current device, without a Stream object or a
+# device switch where torch has these
+_raw_stream = (getattr(torch._C, "_cuda_getCurrentRawStream", None)
+               or (lambda index: torch.cuda.current_stream(index).cuda_stream))
+_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch._C._cuda_getCurrentRawStream(t.device.index)
+    return _raw_stream(t.device.index)
 
 
 class _Here:
@@ -293,7 +304,7 @@ _HERE = _Here()
 
 def on_device(device: torch.device):
     """``torch.cuda.device(device)``, or nothing when that device is the current one."""
-    return _HERE if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
+    return _HERE if _current_device() == device.index else torch.cuda.device(device)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
