@@ -99,8 +99,9 @@ struct BwdParams {
   // row-block kernel): entries row_vals[row_ptr[r] .. row_ptr[r + 1]) of row r
   const int32_t* row_ptr;
   const int32_t* row_vals;
-  // every Q / D row starts below 2^32 16-byte units from the first, and the
-  // gradient rows are whole 16-byte chunks: the 16-bytes-a-lane kernels apply
+  // every Q / D row starts less than 2^32 16-byte units after the first (of a packed
+  // side: after row cu_seqlens[0]), and the gradient rows are whole 16-byte
+  // chunks: the 16-bytes-a-lane kernels apply
   bool q_units, d_units;
 };
 
@@ -850,6 +851,10 @@ __global__ void __launch_bounds__(256) grad_q_rows_kernel(const BwdParams bp) {
     ue = ub + bp.qchunk < nu ? ub + bp.qchunk : nu;
   }
   const bool live = q * 8 < bp.dim;
+  // Offsets count from the first row of the documents: of a packed buffer the
+  // call may use a part that starts anywhere in it.
+  const int64_t d_row0 = bp.d_cu ? (int64_t)bp.d_cu[0] : 0;
+  const char* const d_base = bp.d + d_row0 * bp.d_sl;
   auto load_units = [&](int64_t c0, uint32_t& off, float& sc) {
     off = kNoRow;
     sc = 0.f;
@@ -870,7 +875,7 @@ __global__ void __launch_bounds__(256) grad_q_rows_kernel(const BwdParams bp) {
     }
     if (a < 0 || g == 0.f) return;
     sc = bp.dinv ? g * bp.dinv[jd * bp.ld + a] : g;  // dinv only for padded docs
-    const int64_t b = bp.d_cu ? ((int64_t)bp.d_cu[jd] + a) * bp.d_sl : jd * bp.d_sn + (int64_t)a * bp.d_sl;
+    const int64_t b = bp.d_cu ? ((int64_t)bp.d_cu[jd] - d_row0 + a) * bp.d_sl : jd * bp.d_sn + (int64_t)a * bp.d_sl;
     off = (uint32_t)(b >> 4);
   };
   float acc[8];
@@ -889,7 +894,7 @@ __global__ void __launch_bounds__(256) grad_q_rows_kernel(const BwdParams bp) {
         const uint32_t o = row_bcast<DPL, l>(off);
         cs[k] = __uint_as_float(row_bcast<DPL, l>(__float_as_uint(sc)));
         v[k] = u32x4{0u, 0u, 0u, 0u};
-        if (o != kNoRow && live) v[k] = *(const u32x4*)(bp.d + ((uint64_t)o << 4) + q * 16);
+        if (o != kNoRow && live) v[k] = *(const u32x4*)(d_base + ((uint64_t)o << 4) + q * 16);
       };
       one(std::integral_constant<int, 0>{});
       one(std::integral_constant<int, 1>{});
@@ -1359,9 +1364,13 @@ static size_t grad_q_part_bytes(const lik_seqs_t* Q, const lik_seqs_t* D, uint32
 
 // Whether the 16-bytes-a-lane kernels can address this side's rows: 16-bit rows
 // of up to 128 dims (whole 16-byte chunks; checked by the callers), each
-// starting below 2^32 16-byte units. A packed side has at most n * len rows.
+// starting less than 2^32 16-byte units after the first. A packed side has at
+// most n * len rows from cu_seqlens[0] on. (A packed side whose longest length is
+// not known, len 0, as the decoded documents of a PLAID gradient are, has no such
+// bound and keeps the one-wavefront-per-row kernel.)
 static bool row_units(const lik_seqs_t* x) {
   if ((x->dtype != LIK_BF16 && x->dtype != LIK_F16) || x->dim > 128 || x->n <= 0 || x->len <= 0) return false;
+  if (x->stride_l < 0 || (!x->cu_seqlens && x->stride_n < 0)) return false;
   const int64_t last = x->cu_seqlens ? x->n * x->len * x->stride_l
                                      : (x->n - 1) * x->stride_n + (x->len - 1) * x->stride_l;
   return last >= 0 && last * 2 < ((int64_t)0xffffffff << 4);
