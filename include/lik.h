@@ -377,7 +377,8 @@ int lik_plaid_approx_score(const float* qcs, int64_t n_centroids, int64_t lq, in
  * (scores[r*ld + c], idx_base + c) for c < n. Writes the k best, ordered by
  * score (descending if largest, else ascending) and then by lower index,
  * to out_scores/out_idx[r*out_ld + i]. k <= prev_k + n, k <= 8192,
- * indices < 2^32. For k <= 1024: prev_k <= 1024 and n <= 4096; for larger k:
+ * indices < 2^32; a (score, index) that appears twice counts twice. For
+ * k <= 1024: prev_k <= 1024 and n <= 4096; for larger k:
  * prev_k <= 8192 and n <= 8192. prev may alias out.
  * Replaces the torch.topk + cat + gather merge of topk.py:41-86 /
  * retrieve.py:278-305 with a deterministic tie order (lower index first).

@@ -4,9 +4,10 @@
 //   key = order(score) << 32 | ~index
 // where order() is the monotone float->uint32 map (descending scores map to
 // descending keys; for largest=False the score part is complemented). Keys
-// are unique and never 0 (indices stay below 2^32 - 1), and "larger key" ==
-// "better score, then lower index", so the k best candidates are exactly the
-// k largest keys and any grouping of the candidates selects the same set.
+// are never 0 (indices stay below 2^32 - 1), and "larger key" == "better score,
+// then lower index", so the k best candidates are exactly the k largest keys and
+// any grouping of the candidates selects the same ones. Distinct candidates have
+// distinct keys; one that appears twice counts twice.
 //
 // One workgroup selects the kk largest of up to MAX_KEYS LDS-resident keys by
 // histogram passes of 2048 bins over the keys' own range (then over the bin that
@@ -250,14 +251,18 @@ __global__ void __launch_bounds__(TK_THREADS) topk_select_kernel(TopkArgs a) {
       __syncthreads();
       lo = s_lo;
       kk = (uint32_t)s_kk;
-      if (s_done || shift == 0) break;  // (at shift 0 a bin holds one key: keys are unique)
+      if (s_done || shift == 0) break;  // (at shift 0 a bin holds one key value)
       const int next = shift > TK_BIN_BITS ? shift - TK_BIN_BITS : 0;
       nbins = 1ull << (shift - next);
       shift = next;
     }
 
-    // winners: key >= lo; exactly kk_sel of them (keys are unique and the
-    // kk_sel-th largest is a real key, above every 0 pad)
+    // Winners: key >= lo, exactly kk_sel of them (the kk_sel-th largest is a real
+    // key, above every 0 pad). A candidate given twice (a window merged again over
+    // the running list) is two equal keys: where only kk of the keys equal to lo
+    // belong, the winners are the keys above lo, and kk copies of lo.
+    const bool cut = s_done == 0;
+    const uint64_t from = cut ? lo + 1 : lo;
     if constexpr (C::INPLACE) {
       // In place, one 256-key chunk at a time: every key of the chunk is read
       // before any write, and a winner's slot is below the number of keys
@@ -266,7 +271,7 @@ __global__ void __launch_bounds__(TK_THREADS) topk_select_kernel(TopkArgs a) {
       for (int i0 = 0; i0 < total; i0 += TK_THREADS) {
         const int i = i0 + tid;
         const uint64_t key = i < total ? s_keys[i] : 0;
-        const bool win = i < total && key >= lo;
+        const bool win = i < total && key >= from;
         const uint64_t bal = __ballot(win);
         if (lane == 0) s_wcnt[wv] = (int)__popcll(bal);
         __syncthreads();
@@ -283,12 +288,14 @@ __global__ void __launch_bounds__(TK_THREADS) topk_select_kernel(TopkArgs a) {
     } else {
       for (int i = tid; i < total; i += TK_THREADS) {
         const uint64_t key = s_keys[i];
-        if (key >= lo) {
+        if (key >= from) {
           const int pos = atomicAdd(&s_cnt, 1);
           if (pos < C::MAX_K) s_sel[pos] = key;
         }
       }
     }
+    if (cut)  // (in place: the loop above ended with a barrier, and wrote below these)
+      for (int i = kk_sel - (int)kk + tid; i < kk_sel; i += TK_THREADS) s_sel[i] = lo;
   }
   __syncthreads();
   auto put = [&](int64_t at, uint64_t key) {
@@ -304,12 +311,13 @@ __global__ void __launch_bounds__(TK_THREADS) topk_select_kernel(TopkArgs a) {
   if (a.keys_out)
     for (int i = kk_sel + tid; i < a.k; i += TK_THREADS) put(i, 0);
   if (kk_sel <= TK_THREADS) {
-    // a winner's place is the number of larger ones (the reads are broadcasts)
+    // a winner's place is the number of larger ones and of equal ones before it
+    // (the reads are broadcasts)
     if (tid < kk_sel) {
       const uint64_t key = s_sel[tid];
       int rank = 0;
 #pragma unroll 8
-      for (int i = 0; i < kk_sel; ++i) rank += s_sel[i] > key ? 1 : 0;
+      for (int i = 0; i < kk_sel; ++i) rank += (s_sel[i] > key || (s_sel[i] == key && i < tid)) ? 1 : 0;
       put(rank, key);
     }
     return;
