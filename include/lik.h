@@ -412,6 +412,9 @@ int lik_topk_select(const float* scores, int64_t rows, int64_t n, int64_t ld, in
  */
 int lik_seqlens_cover(const int32_t* cu_a, int64_t n_a, int64_t max_a, const int32_t* cu_b, int64_t n_b, int64_t max_b,
                       uint8_t* ok, lik_stream_t stream);
+/* The same with an answer for each array: *ok_a and *ok_b (both required). */
+int lik_seqlens_cover_each(const int32_t* cu_a, int64_t n_a, int64_t max_a, const int32_t* cu_b, int64_t n_b,
+                           int64_t max_b, uint8_t* ok_a, uint8_t* ok_b, lik_stream_t stream);
 
 /*
  * Projection-head gradients of maxsim_from_hidden training: from grad_d

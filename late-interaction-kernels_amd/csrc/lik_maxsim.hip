@@ -193,22 +193,27 @@ __global__ void __launch_bounds__(256) norm_rows_kernel(const char* x, int64_t s
   *(u32x4*)(out + r * (int64_t)dim * 2 + (int64_t)cc * 16) = v;
 }
 
-// *ok = no sequence of cu_a (cu_b) is longer than max_a (max_b): one workgroup,
-// four sequences per thread and step (9216 sequences: 4 us, against 35 us for
-// the six launches of torch's subtractions, maxima and comparisons).
+// *ok_a (*ok_b) = no sequence of cu_a (cu_b) is longer than max_a (max_b); without
+// ok_b, *ok_a answers for both: one workgroup, four sequences per thread and step
+// (9216 sequences: 4 us, against 35 us for the six launches of torch's
+// subtractions, maxima and comparisons).
 __global__ void __launch_bounds__(1024) seqlens_cover_kernel(const int32_t* cu_a, int64_t n_a, int64_t max_a,
                                                              const int32_t* cu_b, int64_t n_b, int64_t max_b,
-                                                             uint8_t* ok) {
-  bool bad = false;
+                                                             uint8_t* ok_a, uint8_t* ok_b) {
   auto scan = [&](const int32_t* cu, int64_t n, int64_t most) {
+    bool bad = false;
 #pragma unroll 4
     for (int64_t k = threadIdx.x; k < n; k += 1024)
       bad |= (int64_t)(int32_t)((uint32_t)cu[k + 1] - (uint32_t)cu[k]) > most;
+    return bad;
   };
-  scan(cu_a, n_a, max_a);
-  scan(cu_b, n_b, max_b);
-  const int any = __syncthreads_or(bad ? 1 : 0);
-  if (threadIdx.x == 0) *ok = any ? 0 : 1;
+  const bool bad_a = scan(cu_a, n_a, max_a), bad_b = scan(cu_b, n_b, max_b);
+  const int any_a = __syncthreads_or((bad_a || (!ok_b && bad_b)) ? 1 : 0);
+  const int any_b = __syncthreads_or(bad_b ? 1 : 0);
+  if (threadIdx.x == 0) {
+    *ok_a = any_a ? 0 : 1;
+    if (ok_b) *ok_b = any_b ? 0 : 1;
+  }
 }
 
 // out[q, j] = sum_c part[q*nc + c, j], c ascending.
@@ -866,6 +871,13 @@ void* device_scratch(hipStream_t s) {
   return g_scratch_ptr[dev];
 }
 
+int launch_seqlens_cover(const int32_t* cu_a, int64_t n_a, int64_t max_a, const int32_t* cu_b, int64_t n_b,
+                         int64_t max_b, uint8_t* ok_a, uint8_t* ok_b, hipStream_t s) {
+  if (n_a < 0 || n_b < 0 || !ok_a || (n_a > 0 && !cu_a) || (n_b > 0 && !cu_b)) return LIK_ERR_INVALID;
+  hipLaunchKernelGGL(seqlens_cover_kernel, dim3(1), dim3(1024), 0, s, cu_a, n_a, max_a, cu_b, n_b, max_b, ok_a, ok_b);
+  return hipGetLastError() == hipSuccess ? LIK_OK : LIK_ERR_LAUNCH;
+}
+
 }  // namespace
 
 
@@ -875,10 +887,13 @@ const char* lik_version(void) { return "lik-hip 0.1.0 gfx950"; }
 
 int lik_seqlens_cover(const int32_t* cu_a, int64_t n_a, int64_t max_a, const int32_t* cu_b, int64_t n_b, int64_t max_b,
                       uint8_t* ok, lik_stream_t stream) {
-  if (n_a < 0 || n_b < 0 || !ok || (n_a > 0 && !cu_a) || (n_b > 0 && !cu_b)) return LIK_ERR_INVALID;
-  hipLaunchKernelGGL(seqlens_cover_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, cu_a, n_a, max_a, cu_b, n_b,
-                     max_b, ok);
-  return hipGetLastError() == hipSuccess ? LIK_OK : LIK_ERR_LAUNCH;
+  return launch_seqlens_cover(cu_a, n_a, max_a, cu_b, n_b, max_b, ok, nullptr, (hipStream_t)stream);
+}
+
+int lik_seqlens_cover_each(const int32_t* cu_a, int64_t n_a, int64_t max_a, const int32_t* cu_b, int64_t n_b,
+                           int64_t max_b, uint8_t* ok_a, uint8_t* ok_b, lik_stream_t stream) {
+  if (!ok_b) return LIK_ERR_INVALID;
+  return launch_seqlens_cover(cu_a, n_a, max_a, cu_b, n_b, max_b, ok_a, ok_b, (hipStream_t)stream);
 }
 
 size_t lik_maxsim_workspace_size_ex(const lik_seqs_t* Q, const lik_seqs_t* D, uint32_t flags,

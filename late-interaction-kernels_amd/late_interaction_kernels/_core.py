@@ -370,28 +370,27 @@ def assert_max_seqlens_cover(*checks: tuple[torch.Tensor, int | None, str]) -> N
     """On-device check that caller-supplied bounds cover every sequence of one or
     two ``cu_seqlens`` (``_utils.py:32-50``): a bound sizes the query block, so a
     too-small value would drop tokens. One kernel reads both arrays
-    (``lik_seqlens_cover``); the differences, maximum and comparison as torch
-    operators are three launches for each."""
+    (``lik_seqlens_cover_each``), and each bound has its own assert; the
+    differences, maximum and comparison as torch operators are three launches
+    for each."""
     todo = [(cu, m, name) for cu, m, name in checks if m is not None and cu.numel() > 1]
     if not todo:
         return
+    passed = None
     if (len(todo) <= 2 and sum(cu.numel() for cu, _, _ in todo) <= _COVER_MAX
             and all(cu.device == todo[0][0].device and cu.dtype == torch.int32 and cu.is_contiguous()
                     and abs(m) < 1 << 62 for cu, m, _ in todo)
             and _lib.plain_op(*(cu for cu, _, _ in todo))):
-        ok = torch.empty((), device=todo[0][0].device, dtype=torch.bool)
+        ok = torch.empty(2, device=todo[0][0].device, dtype=torch.bool)
         (a, ma, _), (b, mb, _) = todo[0], todo[-1]
         with _lib.on_device(ok.device):
-            rc = _lib.load().lik_seqlens_cover(a.data_ptr(), a.numel() - 1, ma, b.data_ptr(), b.numel() - 1, mb,
-                                               ok.data_ptr(), _lib.stream_of(ok))
-        _lib.check(rc, "lik_seqlens_cover")
-        names = " or ".join(f"{name}={m}" for _, m, name in todo)
-        torch._assert_async(ok, f"{names} is smaller than the longest sequence in cu_seqlens; "
-                            "it is a hard bound and would silently truncate tokens.")
-        return
-    for cu, m, name in todo:
+            rc = _lib.load().lik_seqlens_cover_each(a.data_ptr(), a.numel() - 1, ma, b.data_ptr(), b.numel() - 1, mb,
+                                                    ok.data_ptr(), ok.data_ptr() + 1, _lib.stream_of(ok))
+        _lib.check(rc, "lik_seqlens_cover_each")
+        passed = ok.unbind(0)
+    for k, (cu, m, name) in enumerate(todo):
         torch._assert_async(
-            (cu[1:] - cu[:-1]).max().le(m),
+            (cu[1:] - cu[:-1]).max().le(m) if passed is None else passed[k],
             f"{name}={m} is smaller than the longest sequence in cu_seqlens; "
             "it is a hard bound and would silently truncate tokens.",
         )

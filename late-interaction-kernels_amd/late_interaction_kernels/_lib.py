@@ -79,6 +79,7 @@ EXPORTED_SYMBOLS = (
     "lik_quantize_fp8",
     "lik_quantize_fp8_workspace_size",
     "lik_seqlens_cover",
+    "lik_seqlens_cover_each",
 )
 
 _p = ctypes.c_void_p
@@ -235,6 +236,8 @@ def load() -> ctypes.CDLL:
     lib.lik_head_backward.restype = ctypes.c_int
     lib.lik_seqlens_cover.argtypes = [_p, _i64, _i64, _p, _i64, _i64, _p, _p]
     lib.lik_seqlens_cover.restype = ctypes.c_int
+    lib.lik_seqlens_cover_each.argtypes = [_p, _i64, _i64, _p, _i64, _i64, _p, _p, _p]
+    lib.lik_seqlens_cover_each.restype = ctypes.c_int
     lib.lik_quantize_fp8_workspace_size.argtypes = [ctypes.c_uint32]
     lib.lik_quantize_fp8_workspace_size.restype = ctypes.c_size_t
     lib.lik_quantize_fp8.argtypes = [_p, _i32, _i64, _i32, ctypes.c_uint32, _p, _p, _p, ctypes.c_size_t, _p]

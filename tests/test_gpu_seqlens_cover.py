@@ -47,3 +47,39 @@ def test_bounds_accepted_on_every_entry_point():
     s = score_pairs_packed(Q, D, cq, cd, i.sort().values, i, max_seqlen_q=27, max_seqlen_d=100)
     assert torch.allclose(s.view(3, 3), want, rtol=1e-6, atol=1e-5)  # another order of the column sum
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("entry", ["varlen", "pairs"])
+@pytest.mark.parametrize("mq,md,want", [(27, 100, set()), (26, 100, {"max_seqlen_q=26"}), (27, 99, {"max_seqlen_d=99"}),
+                                        (1, 2, {"max_seqlen_q=1", "max_seqlen_d=2"}), (None, 99, {"max_seqlen_d=99"}),
+                                        (26, None, {"max_seqlen_q=26"})])
+def test_each_bound_has_its_own_message(monkeypatch, entry, mq, md, want):
+    """The assert that fails names the bound that is too small, and no other. (The
+    asserts are recorded on the host here, so none of them fires on the GPU; the
+    calls stop at them.)"""
+    from late_interaction_kernels import maxsim_varlen
+    from late_interaction_kernels.score_pairs import score_pairs_packed
+
+    cq = torch.tensor([0, 5, 5, 32], dtype=torch.int32, device="cuda")
+    cd = torch.tensor([0, 40, 41, 141], dtype=torch.int32, device="cuda")
+    Q, D = torch.zeros(32, 64, device="cuda").bfloat16(), torch.zeros(141, 64, device="cuda").bfloat16()
+    seen = []
+    monkeypatch.setattr(torch, "_assert_async", lambda ok, msg: seen.append((bool(ok), msg)))
+    module = "late_interaction_kernels." + ("varlen" if entry == "varlen" else "score_pairs")
+
+    class Stop(Exception):
+        pass
+
+    def stop(*a, **k):
+        raise Stop
+
+    monkeypatch.setattr(f"{module}.unify_dtype", stop)
+    i = torch.zeros(1, device="cuda", dtype=torch.int32)
+    with pytest.raises(Stop):
+        if entry == "varlen":
+            maxsim_varlen(Q, D, cq, cd, mq, md)
+        else:
+            score_pairs_packed(Q, D, cq, cd, i, i, max_seqlen_q=mq, max_seqlen_d=md)
+    failed = {msg.split(" ")[0] for ok, msg in seen if not ok}
+    assert failed == want
+    assert all(msg.count("max_seqlen") == 1 for _, msg in seen)
