@@ -13,10 +13,11 @@
 // histogram passes of 2048 bins over the keys' own range (then over the bin that
 // holds the kk-th largest), compacts the winners and puts each at its rank (up
 // to 256 of them; more are bitonic-sorted). Latency is what bounds it: a
-// barrier per step and few keys per thread. (Byte-wise passes from the top, whose
-// first ones put all scores of a call in one bin, and a bitonic sort took 17.3 us
-// for 16 rows of 4096 scores at k = 100, 25 + 20 us for the two levels of 100,000
-// scores; now 13.8, and 19 + 12.) A row wider than one workgroup's share is
+// barrier per step and few keys per thread; with many rows, how many workgroups
+// share a CU. (A call with byte-wise passes from the top, whose first ones put all
+// scores of a call in one bin, and a bitonic sort took 19.2 us for 16 rows of 4096
+// scores at k = 100, 33.8 for 100,000 scores, 94.6 for 512 rows of 20,000; now
+// 15.9, 25.5 and 74.6.) A row wider than one workgroup's share is
 // reduced as a tree: level 0 gives each MAX_N-score slice of a row its own
 // workgroup, which writes its k best keys (0-padded) to a workspace; each
 // further level merges up to MAX_KEYS / k such lists per workgroup, and the
@@ -31,7 +32,7 @@ namespace lik {
 constexpr int TK_THREADS = 256;
 constexpr int TK_BIN_BITS = 11, TK_BINS = 1 << TK_BIN_BITS;  // of one selection pass
 // Two LDS capacity classes. Small (k <= 1024): 4096 scores per level-0 group
-// plus a running list, winners sorted in their own array (48 KB). Large
+// plus a running list, winners sorted in the histogram's memory (49 KB). Large
 // (k <= 8192): 16384 keys (128 KB, one workgroup per CU), 8192 scores per
 // level-0 group, winners compacted in place into the key array.
 template <int CLS> struct TkCap;
@@ -62,6 +63,33 @@ __device__ __forceinline__ uint64_t make_key(float s, uint32_t idx, int largest)
   return ((uint64_t)o << 32) | (uint64_t)(~idx);
 }
 
+// Lane v of a step: the lane 1, 2, 4, 8 below in its row of 16, then the last
+// lane of the row (of the two rows) below; 0 where there is none.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_below(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, ROWS == 0xf);
+}
+// Inclusive prefix sum over the wavefront's lanes, and the lanes' maximum. (By
+// register moves: a shuffle through the LDS unit costs 100 cycles a step.)
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+  v += dpp_below<0x111, 0xf>(v);
+  v += dpp_below<0x112, 0xf>(v);
+  v += dpp_below<0x114, 0xf>(v);
+  v += dpp_below<0x118, 0xf>(v);
+  v += dpp_below<0x142, 0xa>(v);
+  v += dpp_below<0x143, 0xc>(v);
+  return v;
+}
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+  v = max(v, dpp_below<0x111, 0xf>(v));
+  v = max(v, dpp_below<0x112, 0xf>(v));
+  v = max(v, dpp_below<0x114, 0xf>(v));
+  v = max(v, dpp_below<0x118, 0xf>(v));
+  v = max(v, dpp_below<0x142, 0xa>(v));
+  v = max(v, dpp_below<0x143, 0xc>(v));
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 struct TopkArgs {
   // level 0: scores [rows, n] (row stride ld), doc index = idx_base + column
   const float* scores;
@@ -87,18 +115,26 @@ template <int CLS, bool FROM_KEYS>
 __global__ void __launch_bounds__(TK_THREADS) topk_select_kernel(TopkArgs a) {
   using C = TkCap<CLS>;
   __shared__ uint64_t s_keys[C::MAX_KEYS];
-  __shared__ uint64_t s_sel_own[C::INPLACE ? 1 : C::MAX_K];
-  uint64_t* const s_sel = C::INPLACE ? s_keys : s_sel_own;
-  __shared__ uint32_t s_hist[TK_BINS];
+  // The histogram's memory takes the winners once the selection is over (small
+  // class: 49 KB of LDS, three workgroups per CU; with memory for both it was two,
+  // and 512 rows of 20,000 scores took 73 us at k = 1, 53 now)
+  __shared__ __attribute__((aligned(16))) uint32_t s_hist[TK_BINS];
+  static_assert(C::INPLACE || C::MAX_K * sizeof(uint64_t) <= sizeof(s_hist), "winners fit the histogram's memory");
+  uint64_t* const s_sel = C::INPLACE ? s_keys : (uint64_t*)s_hist;
   __shared__ uint64_t s_lo;
   __shared__ int s_kk, s_done, s_cnt, s_real, s_fcnt;
   __shared__ int s_wcnt[TK_THREADS / 64];
-  __shared__ uint64_t s_wmin[TK_THREADS / 64], s_wmax[TK_THREADS / 64];
+  __shared__ uint64_t s_wmin[TK_THREADS / 64];
+  __shared__ uint32_t s_wtop[TK_THREADS / 64], s_wlow[TK_THREADS / 64];
 
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int64_t row = blockIdx.x / a.groups;
   const int g = (int)(blockIdx.x - row * a.groups);
   if (tid == 0) s_real = 0;
+  constexpr int BPT = TK_BINS / TK_THREADS;  // bins a thread clears and reads
+  u32x4* const my_bins = (u32x4*)&s_hist[TK_BINS - BPT * (tid + 1)];
+#pragma unroll
+  for (int j = 0; j < BPT / 4; ++j) my_bins[j] = u32x4{0u, 0u, 0u, 0u};
   __syncthreads();
 
   int total;
@@ -173,63 +209,73 @@ __global__ void __launch_bounds__(TK_THREADS) topk_select_kernel(TopkArgs a) {
   const int kk_sel = (int)min(a.k, (int64_t)s_real);
 
   if (kk_sel > 0) {
-    // smallest and largest real key
-    uint64_t mn = ~0ull, mx = 0;
-    for (int i = tid; i < total; i += TK_THREADS) {
-      const uint64_t key = s_keys[i];
-      if (key != 0) {
-        mn = key < mn ? key : mn;
-        mx = key > mx ? key : mx;
+    // Passes over the keys in [lo, lo + nbins << shift): lo and shift follow the
+    // keys' own range, so the first pass already spreads them over the bins
+    // (scores of one call share their leading bits). The range is that of the
+    // score words; where all scores are equal, of the index words.
+    auto word_range = [&](int down, uint32_t& mn, uint32_t& mx) {
+      uint32_t top = 0, low = 0;  // largest word, and largest complement
+      for (int i = tid; i < total; i += TK_THREADS) {
+        const uint64_t key = s_keys[i];
+        const uint32_t w = (uint32_t)(key >> down);
+        if (key != 0) {
+          top = w > top ? w : top;
+          low = ~w > low ? ~w : low;
+        }
       }
-    }
+      top = wave_max(top);
+      low = wave_max(low);
+      if (lane == 0) {
+        s_wtop[wv] = top;
+        s_wlow[wv] = low;
+      }
+      __syncthreads();
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      const uint64_t x = __shfl_xor(mn, o), y = __shfl_xor(mx, o);
-      mn = x < mn ? x : mn;
-      mx = y > mx ? y : mx;
+      for (int w = 0; w < TK_THREADS / 64; ++w) {
+        top = s_wtop[w] > top ? s_wtop[w] : top;
+        low = s_wlow[w] > low ? s_wlow[w] : low;
+      }
+      mn = ~low;
+      mx = top;
+    };
+    uint32_t mn, mx;
+    word_range(32, mn, mx);
+    uint64_t lo = (uint64_t)mn << 32, nbins = TK_BINS;
+    int shift = 32;
+    if (mn == mx) {
+      __syncthreads();  // the words in LDS are read
+      uint32_t in, ix;
+      word_range(0, in, ix);
+      lo += in;
+      mn = in;
+      mx = ix;
+      shift = 0;
     }
-    if (lane == 0) {
-      s_wmin[wv] = mn;
-      s_wmax[wv] = mx;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int w = 0; w < TK_THREADS / 64; ++w) {
-      mn = s_wmin[w] < mn ? s_wmin[w] : mn;
-      mx = s_wmax[w] > mx ? s_wmax[w] : mx;
-    }
-    // Passes over the keys in [lo, lo + nbins << shift): lo and shift follow
-    // the keys' own range, so the first pass already spreads them over the
-    // bins (scores of one call share their leading bits).
-    uint64_t lo = mn, nbins = TK_BINS;
-    const uint64_t span = mx - mn;
-    int shift = span ? 64 - __builtin_clzll(span) - TK_BIN_BITS : 0;
-    shift = shift < 0 ? 0 : shift;
+    if (mn != mx) shift += 32 - __builtin_clz(mx - mn);
+    shift = shift < TK_BIN_BITS ? 0 : shift - TK_BIN_BITS;
+    if (lo == 0) lo = 1;  // (0 is no key)
     uint32_t kk = (uint32_t)kk_sel;
     for (;;) {
-      for (int i = tid; i < TK_BINS; i += TK_THREADS) s_hist[i] = 0;
-      __syncthreads();
       for (int i = tid; i < total; i += TK_THREADS) {
         const uint64_t key = s_keys[i];
         const uint64_t bin = (key - lo) >> shift;
         if (key >= lo && bin < nbins) atomicAdd(&s_hist[bin], 1u);
       }
       __syncthreads();
-      // thread t owns 8 bins from TK_BINS - 1 - 8 t down; one of them finds the
-      // bin holding the kk-th largest key of the range
-      constexpr int BPT = TK_BINS / TK_THREADS;
+      // thread t owns 8 bins from TK_BINS - 1 - 8 t down (and clears them for the
+      // next pass); one of them finds the bin holding the kk-th largest key of the range
       uint32_t c[BPT], local = 0;
 #pragma unroll
-      for (int j = 0; j < BPT; ++j) {
-        c[j] = s_hist[TK_BINS - 1 - BPT * tid - j];
-        local += c[j];
-      }
-      uint32_t incl = local;
+      for (int j = 0; j < BPT / 4; ++j) {
+        const u32x4 v = my_bins[j];
+        my_bins[j] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t v = __shfl_up(incl, o);
-        if (lane >= o) incl += v;
+        for (int e = 0; e < 4; ++e) {
+          c[BPT - 1 - 4 * j - e] = v[e];
+          local += v[e];
+        }
       }
+      uint32_t incl = wave_scan(local);
       if (lane == 63) s_wcnt[wv] = (int)incl;
       __syncthreads();
       for (int w = 0; w < wv; ++w) incl += (uint32_t)s_wcnt[w];
@@ -312,12 +358,18 @@ __global__ void __launch_bounds__(TK_THREADS) topk_select_kernel(TopkArgs a) {
     for (int i = kk_sel + tid; i < a.k; i += TK_THREADS) put(i, 0);
   if (kk_sel <= TK_THREADS) {
     // a winner's place is the number of larger ones and of equal ones before it
-    // (the reads are broadcasts)
+    // (the reads are broadcasts; which of the two counts is known for all lanes
+    // outside the wavefront's own 64)
     if (tid < kk_sel) {
       const uint64_t key = s_sel[tid];
+      const int w0 = 64 * __builtin_amdgcn_readfirstlane(wv), w1 = min(w0 + 64, kk_sel);
       int rank = 0;
 #pragma unroll 8
-      for (int i = 0; i < kk_sel; ++i) rank += (s_sel[i] > key || (s_sel[i] == key && i < tid)) ? 1 : 0;
+      for (int i = 0; i < w0; ++i) rank += s_sel[i] >= key ? 1 : 0;
+#pragma unroll 8
+      for (int i = w0; i < w1; ++i) rank += (s_sel[i] > key || (s_sel[i] == key && i < tid)) ? 1 : 0;
+#pragma unroll 8
+      for (int i = w1; i < kk_sel; ++i) rank += s_sel[i] > key ? 1 : 0;
       put(rank, key);
     }
     return;

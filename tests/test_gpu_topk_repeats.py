@@ -64,3 +64,13 @@ def test_padded_running_list(k):
     assert torch.equal(got_s[:, :3], torch.gather(s, 1, order)) and torch.equal(got_i[:, :3], order + 50)
     assert bool((got_s[:, 3:] == float("-inf")).all())
     assert bool((got_i[:, 3:] == 0xFFFFFFFF).all())  # indices are 32-bit (include/lik.h)
+
+
+@pytest.mark.parametrize("k", [3, 200, 700])
+def test_one_candidate_many_times(k):
+    """All candidates equal, the index word of their keys 0 or not."""
+    for index in (-1, 41):
+        s = torch.full((2, 1), float("-inf"), device="cuda")
+        ri = torch.full((2, k), index, device="cuda", dtype=torch.int64)
+        got_s, got_i = _update(s, index & 0xFFFFFFFF, s.expand(2, k).contiguous(), ri, k, True)
+        assert bool((got_s == float("-inf")).all()) and bool((got_i == index & 0xFFFFFFFF).all())
