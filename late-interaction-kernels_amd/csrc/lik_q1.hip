@@ -123,12 +123,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
   }
 
   // ---- doc table of this wavefront's range (empty docs score 0 here) ----
+  auto doc_of = [&](int k) -> int64_t {
+    if (!p.pair_d) return kd_base + jl0 + k;
+    const int64_t pd = p.pair_d[g];
+    return pd >= 0 && pd < p.d.n ? pd : -1;  // out of range: scores 0
+  };
   for (int k = lane; k < nloc; k += 64) {
-    int64_t dg = kd_base + jl0 + k;
-    if (p.pair_d) {
-      const int64_t pd = p.pair_d[g];
-      dg = pd >= 0 && pd < p.d.n ? pd : -1;  // out of range: scores 0
-    }
+    const int64_t dg = doc_of(k);
     const int64_t L = doc_len<SRC_DENSE>(p, dg);
     const bool holed = HOLES && p.holes[dg] != 0;
     int64_t len = L, off = dg < 0 ? 0 : (p.d.cu ? (int64_t)p.d.cu[dg] * p.d.sl_b : dg * p.d.sn_b);
@@ -150,7 +151,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) m
   }
   __builtin_amdgcn_wave_barrier();
   // split: the doc's length and this wavefront's first tile
-  const int64_t dlen = split ? doc_len<SRC_DENSE>(p, kd_base + jl0) : 0;
+  const int64_t dlen = split ? doc_len<SRC_DENSE>(p, doc_of(0)) : 0;
   const int tile0 = split ? (int)((((dlen + 31) >> 5) * wl) >> 2) : 0;
   const float osc = p.out_scale;
 
@@ -504,10 +505,12 @@ int launch_q1(int dt, const Plan& pl, const Params& p0, hipStream_t s) {
   if ((int64_t)p.QPG * p.LU > 32) p.QPG = 32 / p.LU;
   p.R = q1_docs_per_wave(p0);
   p.NR = (p.ndocs_pg + p.R - 1) / p.R;
-  // Few docs (scoring): four wavefronts to each, a serial walk of its tiles being
-  // what such a call waits for (one query, 50 docs of 180 tokens: 14.2 -> 10.6
-  // us); above 512 docs the 2048 wavefronts the chip holds have a doc each.
-  p.split4 = !p.amax && !p.pair_d && p.R == 1 && p.ngroups * p.ndocs_pg <= 512;
+  // Few docs or pairs (scoring): four wavefronts to each, a serial walk of its
+  // tiles being what such a call waits for (one query, 50 docs of 180 tokens: 14.2
+  // -> 10.6 us; pairs with docs of 2048 tokens, d 128: 16 pairs 34 -> 12 us, 256
+  // pairs 44 -> 26, 512 pairs 49 -> 46, where the tile kernel takes 38, 38 and 47);
+  // above 512 docs the 2048 wavefronts the chip holds have a doc each.
+  p.split4 = !p.amax && p.R == 1 && p.ngroups * p.ndocs_pg <= 512;
   const bool normq = (p.normalize & 1) != 0;
   if (pl.dpad == 64)
     return dt == LIK_BF16 ? launch_q1_t<EK_BF16, 64>(p, normq, s) : launch_q1_t<EK_F16, 64>(p, normq, s);

@@ -47,3 +47,29 @@ def test_split_kd_and_nan():
     with launch_options(cfg=(4, 1)):
         assert torch.equal(got, maxsim(Q, D))
     assert got[1, 2] == 0 and torch.isfinite(got).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("P,Lq,Ld,d", [(1, 32, 1, 128), (7, 32, 300, 128), (512, 8, 70, 128), (300, 32, 1030, 64),
+                                       (65, 20, 129, 256), (33, 32, 97, 512), (40, 31, 257, 96)])
+def test_split_pairs_equal_whole_docs(P, Lq, Ld, d, dtype):
+    """Pair lists of up to 512 pairs split their docs too: the bits of the same
+    pairs in a list of more than 512, where a wavefront takes a whole doc."""
+    from late_interaction_kernels.score_pairs import score_pairs_packed
+
+    nq, nd = 5, 40
+    g = torch.Generator(device="cuda").manual_seed(P + Ld)
+    lens = torch.randint(0, Ld + 1, (nd,), generator=g, device="cuda")
+    lens[:3] = torch.tensor([Ld, 0, 1])
+    ql = torch.tensor([Lq, 1, 0, Lq, 5], device="cuda").clamp_max(Lq)
+    cd, cq = (torch.nn.functional.pad(x.cumsum(0), (1, 0)).to(torch.int32) for x in (lens, ql))
+    Q = torch.randn(int(cq[-1]), d, generator=g, device="cuda").to(dtype)
+    D = torch.randn(int(cd[-1]), d, generator=g, device="cuda").to(dtype)
+    D[int(cd[1]) - 1, 3] = float("nan")
+    pq = torch.randint(-1, nq + 1, (P,), generator=g, device="cuda").to(torch.int32)  # ids out of range too
+    pd = torch.randint(-1, nd + 1, (P,), generator=g, device="cuda").to(torch.int32)
+    pq[0], pd[0] = 0, 0
+    times = 512 // P + 1
+    got = score_pairs_packed(Q, D, cq, cd, pq, pd, max_seqlen_q=Lq, max_seqlen_d=Ld)
+    want = score_pairs_packed(Q, D, cq, cd, pq.repeat(times), pd.repeat(times), max_seqlen_q=Lq, max_seqlen_d=Ld)
+    assert torch.equal(got, want[:P]) and torch.isfinite(got).all()
