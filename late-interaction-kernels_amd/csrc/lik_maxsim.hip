@@ -416,32 +416,46 @@ int pick_R(int64_t ngroups, int64_t ndocs, int dpad, const lik_launch_opts_t* op
     const int64_t r1 = (ndocs + wgs - 1) / wgs;
     if (r1 > R) R = r1;
   } else if (ngroups > 1 && wg_cu > 0 && dpad > 0 && dpad <= 128) {
-    // Several query blocks: a workgroup costs ~11 us of query-block load and
-    // pipeline fill, as much as 8 tiles, so the docs are dealt out in whole
-    // rounds of the chip: with k doc ranges per XCD, k * ngroups workgroups
-    // share its 32 * wg_cu slots. Of 1 .. 16 rounds (k as large as they allow)
-    // the cheapest, counting the rounds' tiles and fills and, for the uneven end
-    // of the last one, a tenth of a workgroup's tiles. (Packed corpora keep ~2048
-    // workgroups: lengths that vary a hundredfold need more, shorter workgroups,
-    // by how much only the lengths tell: 33 queries x 500 docs of 16 to 2048
-    // tokens 128 us, this rule's 168 workgroups 171.) Against ~2048 workgroups
-    // whatever the size: 256 x 32 query tokens, 256 docs of 50 to 300 tokens 131 -> 93 us
+    // Several query blocks: the docs are dealt out so that every CU gets the
+    // same number of workgroups. With k doc ranges per XCD its 32 CUs share
+    // k * ngroups workgroups, the fullest one n = ceil(k * ngroups / 32) of them,
+    // wg_cu at a time: of the k for which that is at most 16 times wg_cu, the
+    // cheapest. In units of 3/4 tile (padded docs are part masked) a range costs
+    // its tiles, 0.8 of them where two workgroups share the CU; each load of
+    // query blocks and pipeline fill 21; the uneven end 0.14 of a range and, for
+    // lengths that vary, 0.9 tiles of a doc times the root of the range's docs.
+    // The constants are fitted to 770 measured shapes (20 to 500 queries, 40 to
+    // 2000 docs of 100 to 2048 tokens; bf16 d 128, fp16 d 64, fp32, fp8, the
+    // training block, 300-token queries): within 3% of the best range on average
+    // (~2048 workgroups whatever the size: 28%), and of 653 shapes of uniform or
+    // evenly spread lengths one is more than 3% slower than with ~2048
+    // workgroups. (Whole rounds of all wg_cu slots, as if a second workgroup on
+    // a CU were free: 11, for instance 100 x 100 docs of 1030 tokens, fp16 d 64:
+    // 2 docs in a workgroup 128 us, 1 doc 108.) Padded docs of lengths that vary a
+    // hundredfold remain a gamble on the masks: from 17% slower (training, 64
+    // queries x 256 docs, d 64) to 30% faster (256 queries x 40 docs). (Packed corpora keep ~2048 workgroups: 33 queries x 500 docs
+    // of 16 to 2048 tokens 128 us, 168 workgroups 171.) Against ~2048
+    // workgroups: 256 x 32 query tokens, 256 docs of 50 to 300 tokens 131 -> 93 us
     // (training forward 239 -> 153), 64 queries x 1000 docs 172 -> 96, fp8 64 x 24
     // tokens x 1000 pages 265 -> 223, fp32 32 queries x 2048 docs 464 -> 315; 512 x
-    // 4096 docs at 16 docs per workgroup 2176 us, 32: 2150, 64: 2135, 128: 2126.
-    const int64_t slots = 32 * wg_cu;
-    const double tiles = (double)((len + 31) / 32) * 0.75;  // per doc, part of them masked
+    // 4096 docs take 64 docs per workgroup either way.
+    const double tiles = (double)((len + 31) / 32) * 0.75;
     double best = 0.0;
-    const int64_t r0 = (ngroups + slots - 1) / slots;
-    for (int64_t r = r0; r < r0 + 16; ++r) {
-      const int64_t k = r * slots / ngroups;
-      const int64_t docs = (ndocs + 8 * k - 1) / (8 * k);
-      const double cost = r * (docs * tiles + 8.0) + 0.1 * docs * tiles;
-      if (r == r0 || cost < best) {
+    for (int64_t r = 0; r != 1;) {
+      const bool first = r == 0;
+      const int64_t most = first ? 512 : r - 1;  // docs a range may have
+      const int64_t k = (ndocs + 8 * most - 1) / (8 * most);
+      r = (ndocs + 8 * k - 1) / (8 * k);
+      const int64_t nr = (ndocs + r - 1) / r;
+      const int64_t n = nr >= 8 ? ((nr + 7) / 8 * ngroups + 31) / 32 : (nr * ngroups + 255) / 256;
+      if (!first && n > 16 * wg_cu) break;
+      const double range = r * tiles;
+      const double cost = n * range * (wg_cu > 1 && n > 1 ? 0.8 : 1.0) + (double)((n + wg_cu - 1) / wg_cu) * 21.0 +
+                          0.14 * range + 0.9 * sqrt((double)r) * tiles;
+      if (first || cost < best) {
         best = cost;
-        R = docs;
+        R = r;
       }
-      if (docs <= 1) break;
     }
   }
   if (opts && opts->docs_per_wg > 0) R = opts->docs_per_wg;  // caller-forced (lik_launch_opts_t)
