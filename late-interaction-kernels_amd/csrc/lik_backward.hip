@@ -943,8 +943,8 @@ __global__ void __launch_bounds__(256) grad_q_rows_kernel(const BwdParams bp) {
 // (grad_d_sorted_kernel, which more pairs still take) this is one launch that
 // reads the argmax once and writes nothing but the gradient: 8192 pairs per
 // doc, 256 docs of 300 rows: 215 us in 12 launches -> 43 us. 2048 pairs and
-// fewer run four-wavefront workgroups, several per CU; above 12288 pairs the
-// sorted entries (8 bytes each) no longer fit the LDS beside the counters.
+// fewer run four-wavefront workgroups, several per CU. 12288 pairs are 12 a
+// thread, 132 KB of LDS; it would hold 15360 beside the counters, not 16384.
 template <int EK, int DPL, int NW, int MAXP, int MAXROWS>
 __global__ void __launch_bounds__(NW * 64) grad_d_doc_kernel(const BwdParams bp, int nsplit, int rows_per) {
   constexpr int NT = NW * 64, CH = MAXP / NT, RPT = (MAXROWS + NT - 1) / NT, LPR = 8 * DPL;

@@ -534,11 +534,14 @@ bool prenorm_docs(const lik_seqs_t* Q, const lik_seqs_t* D, uint32_t flags, cons
 // The plan of a scoring call: the two-workgroup 4 x 4 block (fp8 also 4 x 6)
 // is preferred when the tile loop does no doc-side work (no doc normalise left
 // in the kernel, no argmax). fp8 rows with their own scales count as plain at
-// 65 .. 128 dims, where the kernel is compiled for exactly that: the scales
-// cost one multiply per element of the epilogue (64 x 24 query tokens against
-// 1000 x 1030 rows of d = 128: 494 us on 8 x 4, which also left a third of its
-// second 1024-column group empty, 239 us on 4 x 6). At other widths the
-// all-features kernel takes one workgroup per CU either way and keeps 8 x 4.
+// 65 .. 128 dims: the scales cost one multiply per element of the epilogue (64 x 24
+// query tokens against 1000 x 1030 rows of d = 128: 494 us on 8 x 4, which also
+// left a third of its second 1024-column group empty, 239 us on 4 x 6). Only the
+// scales' own kernel runs two workgroups per CU; masks with holes take the
+// all-features kernel, one per CU, and are still faster on 4 x 6 than on 8 x 4 (all
+// docs with holes 574 -> 478 us, half of them 1024 -> 359; 128 x 32 query tokens x
+// 1000 docs of 300: 491 -> 464). At other widths it is that kernel for every call,
+// and 8 x 4 stays.
 int plan_call(const lik_seqs_t* Q, const lik_seqs_t* D, uint32_t flags, bool argmax, Plan& pl, bool& prenorm,
               const lik_launch_opts_t* opts, bool allow_prenorm = true) {
   const bool kd = (flags & LIK_KD_LAYOUT) != 0;
