@@ -68,9 +68,10 @@ def test_padded_running_list(k):
 
 @pytest.mark.parametrize("k", [3, 200, 700])
 def test_one_candidate_many_times(k):
-    """All candidates equal, the index word of their keys 0 or not."""
+    """A full list of one candidate, the index word of its key 0 or not, and a
+    window below it: all the keys that are compared are equal."""
     for index in (-1, 41):
-        s = torch.full((2, 1), float("-inf"), device="cuda")
+        s = torch.full((2, 5), float("-inf"), device="cuda")
         ri = torch.full((2, k), index, device="cuda", dtype=torch.int64)
-        got_s, got_i = _update(s, index & 0xFFFFFFFF, s.expand(2, k).contiguous(), ri, k, True)
-        assert bool((got_s == float("-inf")).all()) and bool((got_i == index & 0xFFFFFFFF).all())
+        got_s, got_i = _update(s, 50, torch.zeros(2, k, device="cuda"), ri, k, True)
+        assert bool((got_s == 0).all()) and bool((got_i == index & 0xFFFFFFFF).all())
